@@ -167,8 +167,6 @@ struct nf3d_engine {
   // region_psd scratch (kept apart from the engine's own pattern estimate)
   float2* d_rspec = nullptr;
   float* d_rsums = nullptr;
-  int* d_rchoice = nullptr;
-  float* d_rglobal = nullptr;
   // staging for host-fed planes
   std::vector<uint8_t*> d_stage;
   std::vector<int> stage_frame;
@@ -259,8 +257,6 @@ struct nf3d_engine {
     hipFree(d_rpat3d);
     hipFree(d_rspec);
     hipFree(d_rsums);
-    hipFree(d_rchoice);
-    hipFree(d_rglobal);
     for (auto* p : d_stage) hipFree(p);
     hipFree(d_dst);
     for (auto ev : ev_pool) hipEventDestroy(ev);
@@ -764,8 +760,8 @@ struct nf3d_engine {
   }
 
   // The per-region noise patterns of one plane as a per-block PSD: the
-  // plane's analysis, the plane-wide search (the fallback of regions without
-  // a searchable block), then each region's own search and its block's
+  // plane's analysis, the blocks' sums, then each region's own search (the
+  // plane's for a region without a searchable block) and its block's
   // |X - degrid correction|^2 x pattern window written to every block of the
   // region (src/helper.cpp:46-132, region by region).  Leaves the engine's
   // own pattern untouched.
@@ -773,8 +769,6 @@ struct nf3d_engine {
     if (!d_rspec) {
       d_rspec = dev_alloc<float2>(spec_elems);
       d_rsums = dev_alloc<float>(nb);
-      d_rchoice = dev_alloc<int>(2);
-      d_rglobal = dev_alloc<float>((size_t)ep.bh * outwidth);
     }
     PlaneJob J = base_job();
     J.src = src;
@@ -790,13 +784,9 @@ struct nf3d_engine {
     P.grid = d_grid;
     P.pwin = d_pwin;
     P.degrid = ep.degrid;
-    P.px = 0;
-    P.py = 0;
-    P.pattern2d = d_rglobal;
     P.sums = d_rsums;
-    P.choice = d_rchoice;
     check(nf3d::launch_pattern(P, s), "pattern kernels");
-    check(nf3d::launch_pattern_regions(P, rx, ry, out, out, 1.0f, s), "region pattern kernel");
+    check(nf3d::launch_pattern_regions(P, rx, ry, out, nullptr, 1.0f, s), "region pattern kernel");
   }
 
   void ensure_pattern3d(int btcur, hipStream_t s) {

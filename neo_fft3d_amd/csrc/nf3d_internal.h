@@ -124,7 +124,7 @@ struct PatternJob {
   int px, py;          // fixed block, or 0,0 = search
   float* pattern2d;    // out [bh*outwidth]
   float* sums;         // scratch [nb]
-  int* choice;         // out [2]: px, py
+  int* choice;         // out [2]: px, py (null: the sums alone)
 };
 
 // Launchers; return hipSuccess or the launch error.  `bw`/`bh` select the
@@ -134,8 +134,9 @@ hipError_t launch_tile(int mode, int bt, int onchip, int mf, int bw, int bh, con
 // Block shapes with a matrix-core DFT variant of k_tile (mf = 1).
 bool mfma_dft_supported(int bw, int bh);
 hipError_t launch_pattern(const PatternJob& job, hipStream_t s);
-// Per-region patterns after launch_pattern (which fills sums and choice):
-// every block gets its rx x ry region's pattern, 2D and times mult3d.
+// Per-region patterns after launch_pattern (which fills sums, and choice if given):
+// every block gets its rx x ry region's pattern, 2D and times mult3d (out3d
+// null: the 2D one alone).
 hipError_t launch_pattern_regions(const PatternJob& job, int rx, int ry, float* out2d, float* out3d, float mult3d,
                                   hipStream_t s);
 // DFT-as-GEMM precision form (nf3d_mfma_dft.hip): n x n blocks, n = 32 or 64.

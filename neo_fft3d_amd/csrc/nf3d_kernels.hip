@@ -7,56 +7,141 @@
 namespace nf3d {
 
 // ----------------------------------------------------------------- pattern
-// Sum of the windowed, degrid-corrected power of each candidate block, in
-// the reference's sequential float order (src/helper.cpp:57-89).
-__global__ void k_pattern_sums(PatternJob J) {
-#pragma clang fp contract(off)
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  int nb = J.nox * J.noy;
-  if (b >= nb) return;
-  int by = b / J.nox, bx = b - by * J.nox;
-  if (by < 2 || by >= J.noy - 2 || bx < 2 || bx >= J.nox - 2) { J.sums[b] = 3.0e38f; return; }
-  const float2* blk = J.spec + (size_t)b * J.bh * J.outwidth;
-  float gcur = J.degrid * blk[0].x / J.grid[0].x;
-  float s = 0.0f;
-  for (int k = 0; k < J.bh * J.outwidth; k++) {
-    float2 g = J.grid[k];
-    float c0 = blk[k].x - gcur * g.x, c1 = blk[k].y - gcur * g.y;
-    float psd = c0 * c0 + c1 * c1;
-    s += psd * J.pwin[k];
-  }
-  J.sums[b] = s;
+// Blocks of the pattern search (src/helper.cpp:60-63): two blocks of border.
+__device__ __forceinline__ bool pattern_candidate(int nox, int noy, int bx, int by) {
+  return by >= 2 && by < noy - 2 && bx >= 2 && bx < nox - 2;
 }
 
-// First strict minimum in row-major block order, then the pattern of the
-// chosen block (src/helper.cpp:82-88, 111-130).  One workgroup.
+// |X - g G|^2 times the pattern window, one coefficient (src/helper.cpp:66-75).
+__device__ __forceinline__ float pattern_term(float2 c, float2 g, float gcur, float pw) {
+#pragma clang fp contract(off)
+  const float c0 = c.x - gcur * g.x, c1 = c.y - gcur * g.y;
+  const float psd = c0 * c0 + c1 * c1;
+  return psd * pw;
+}
+
+// Sum of the windowed, degrid-corrected power of each candidate block, in
+// the reference's sequential float order (src/helper.cpp:57-89).  A wavefront
+// per block: its 64 lanes read the spectrum, the gridsample and the pattern
+// window row by row of 64 coefficients (coalesced, the next PS_ROWS rows in
+// flight) and leave the terms in LDS; one lane then adds them in order, 16
+// bytes a read.  Bound by that serial chain of bh * (bw/2+1) adds, which the
+// blocks' wavefronts (two to three per SIMD at 1080p) run side by side; with
+// a lane per block instead, every load was a line of its own and the few
+// wavefronts waited for each: 137 us on a 1920x1080 plane's 2,232 blocks of
+// 48x48, now 11.9 us.
+constexpr int PS_CHUNK = 512;             // terms of a block in LDS at a time
+constexpr int PS_ROWS = PS_CHUNK / 64;
+__global__ void __launch_bounds__(64) k_pattern_sums(PatternJob J) {
+#pragma clang fp contract(off)
+  __shared__ __align__(16) float term[PS_CHUNK];
+  const int b = blockIdx.x, l = threadIdx.x;
+  const int by = b / J.nox, bx = b - by * J.nox;
+  if (!pattern_candidate(J.nox, J.noy, bx, by)) {
+    if (l == 0) J.sums[b] = 3.0e38f;
+    return;
+  }
+  const int n = J.bh * J.outwidth;
+  const float2* blk = J.spec + (size_t)b * n;
+  const float gcur = J.degrid * blk[0].x / J.grid[0].x;
+  float2 c[PS_ROWS], g[PS_ROWS];
+  float w[PS_ROWS];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < PS_ROWS; u++) {
+      const int k = min(k0 + u * 64 + l, n - 1);
+      c[u] = blk[k];
+      g[u] = J.grid[k];
+      w[u] = J.pwin[k];
+    }
+  };
+  load(0);
+  float s = 0.0f;
+  for (int k0 = 0; k0 < n; k0 += PS_CHUNK) {
+#pragma unroll
+    for (int u = 0; u < PS_ROWS; u++) term[u * 64 + l] = pattern_term(c[u], g[u], gcur, w[u]);
+    __syncthreads();
+    if (k0 + PS_CHUNK < n) load(k0 + PS_CHUNK);
+    const int m = min(PS_CHUNK, n - k0);
+    int k = 0;
+#pragma unroll 4
+    for (; k + 8 <= m; k += 8) {  // (every lane adds: the same sum)
+      const float4 a = *reinterpret_cast<const float4*>(term + k), d = *reinterpret_cast<const float4*>(term + k + 4);
+      s += a.x;
+      s += a.y;
+      s += a.z;
+      s += a.w;
+      s += d.x;
+      s += d.y;
+      s += d.z;
+      s += d.w;
+    }
+    for (; k < m; k++) s += term[k];
+    __syncthreads();
+  }
+  if (l == 0) J.sums[b] = s;
+}
+
+// The first strict minimum below 1e15 of the sums of the search range's
+// blocks in [x0, x1) x [y0, y1), in row-major order (src/helper.cpp:82-88):
+// the smallest value, the first block of equal ones.  256 lanes take the
+// blocks in turn and meet in LDS (one lane alone waited for every load:
+// k_pattern_set took 124 us on 1,856 sums, now 6.7 us).  Returns the block's
+// index by * nox + bx, or -1.
+__device__ __forceinline__ int pattern_search(const PatternJob& J, int x0, int x1, int y0, int y1, float* rv, int* ri) {
+  x0 = max(x0, 2);
+  y0 = max(y0, 2);
+  x1 = min(x1, J.nox - 2);
+  y1 = min(y1, J.noy - 2);
+  const int w = max(x1 - x0, 0), n = w * max(y1 - y0, 0), t = threadIdx.x;
+  float best = 1e15f;
+  int at = 0x7fffffff;
+  for (int k = t; k < n; k += 256) {
+    const int y = k / w, i = (y0 + y) * J.nox + x0 + (k - y * w);
+    const float s = J.sums[i];
+    if (s < best) {
+      best = s;
+      at = i;
+    }
+  }
+  __syncthreads();  // (a second search: the first one's result is read)
+  rv[t] = best;
+  ri[t] = at;
+  __syncthreads();
+  int h = 1;
+  while (h < min(n, 256)) h <<= 1;  // lanes past n hold no block
+  for (h >>= 1; h > 0; h >>= 1) {
+    if (t < h && (rv[t + h] < rv[t] || (rv[t + h] == rv[t] && ri[t + h] < ri[t]))) {
+      rv[t] = rv[t + h];
+      ri[t] = ri[t + h];
+    }
+    __syncthreads();
+  }
+  return ri[0] == 0x7fffffff ? -1 : ri[0];
+}
+
+// The searched block, or the given one, and its pattern (src/helper.cpp:
+// 82-88, 111-130).  One workgroup.
 __global__ void __launch_bounds__(256) k_pattern_set(PatternJob J) {
 #pragma clang fp contract(off)
-  __shared__ int choice[2];
-  if (threadIdx.x == 0) {
-    int px = J.px, py = J.py;
-    if (px == 0 && py == 0) {
-      float best = 1e15f;
-      for (int by = 2; by < J.noy - 2; by++)
-        for (int bx = 2; bx < J.nox - 2; bx++) {
-          float s = J.sums[by * J.nox + bx];
-          if (s < best) { best = s; px = bx; py = by; }
-        }
+  __shared__ float rv[256];
+  __shared__ int ri[256];
+  int px = J.px, py = J.py;
+  if (px == 0 && py == 0) {
+    const int i = pattern_search(J, 0, J.nox, 0, J.noy, rv, ri);
+    if (i >= 0) {
+      py = i / J.nox;
+      px = i - py * J.nox;
     }
-    choice[0] = px;
-    choice[1] = py;
+  }
+  if (threadIdx.x == 0) {
     J.choice[0] = px;
     J.choice[1] = py;
   }
-  __syncthreads();
-  const float2* blk = J.spec + ((size_t)choice[1] * J.nox + choice[0]) * J.bh * J.outwidth;
-  float gcur = J.degrid * blk[0].x / J.grid[0].x;
-  for (int k = threadIdx.x; k < J.bh * J.outwidth; k += blockDim.x) {
-    float2 g = J.grid[k];
-    float c0 = blk[k].x - gcur * g.x, c1 = blk[k].y - gcur * g.y;
-    float psd = c0 * c0 + c1 * c1;
-    J.pattern2d[k] = psd * J.pwin[k];
-  }
+  const float2* blk = J.spec + ((size_t)py * J.nox + px) * J.bh * J.outwidth;
+  const float gcur = J.degrid * blk[0].x / J.grid[0].x;
+  for (int k = threadIdx.x; k < J.bh * J.outwidth; k += blockDim.x)
+    J.pattern2d[k] = pattern_term(blk[k], J.grid[k], gcur, J.pwin[k]);
 }
 
 // Spatially varying noise pattern (no reference counterpart; it generalises
@@ -65,47 +150,36 @@ __global__ void __launch_bounds__(256) k_pattern_set(PatternJob J) {
 // pattern of its own first strict minimum of the same sums over the blocks
 // of the reference's search range (blocks 2..nox-3, 2..noy-3) that lie in
 // it -- or, for a region with none of them, the block chosen for the whole
-// plane (J.choice, written by k_pattern_set).  The pattern goes to every
-// block of the region: out2d = |X - g G|^2 pwin, out3d = out2d * mult3d.
-// One workgroup per region.
+// plane (J.choice, written by k_pattern_set; null: searched here, which for
+// the few such regions costs less than a launch of its own, 6.7 us, before
+// this one).  The pattern goes to every
+// block of the region: out2d = |X - g G|^2 pwin, out3d = out2d * mult3d
+// (out3d null: out2d alone).  blockIdx.x: the region, blockIdx.y: 256 of the
+// coefficients (1080p at 48x48 in regions of 4 x 4 has 144 regions, fewer
+// than there are CUs).
 __global__ void __launch_bounds__(256) k_pattern_regions(PatternJob J, int rx, int ry, float* out2d, float* out3d,
                                                          float mult3d) {
 #pragma clang fp contract(off)
-  __shared__ int choice[2];
+  __shared__ float rv[256];
+  __shared__ int ri[256];
   const int nqx = (J.nox + rx - 1) / rx;
   const int qy = blockIdx.x / nqx, qx = blockIdx.x - qy * nqx;
   const int x0 = qx * rx, x1 = min(J.nox, x0 + rx), y0 = qy * ry, y1 = min(J.noy, y0 + ry);
-  if (threadIdx.x == 0) {
-    int px = -1, py = -1;
-    float best = 1e15f;
-    for (int by = max(y0, 2); by < min(y1, J.noy - 2); by++)
-      for (int bx = max(x0, 2); bx < min(x1, J.nox - 2); bx++) {
-        const float v = J.sums[by * J.nox + bx];
-        if (v < best) { best = v; px = bx; py = by; }
-      }
-    if (px < 0) {
-      px = J.choice[0];
-      py = J.choice[1];
-    }
-    choice[0] = px;
-    choice[1] = py;
-  }
-  __syncthreads();
+  int c = pattern_search(J, x0, x1, y0, y1, rv, ri);
+  if (c < 0) c = J.choice ? J.choice[1] * J.nox + J.choice[0] : max(pattern_search(J, 0, J.nox, 0, J.noy, rv, ri), 0);
   const int n = J.bh * J.outwidth;
-  const float2* blk = J.spec + ((size_t)choice[1] * J.nox + choice[0]) * n;
+  const int k = blockIdx.y * 256 + threadIdx.x;
+  if (k >= n) return;
+  const float2* blk = J.spec + (size_t)c * n;
   const float gcur = J.degrid * blk[0].x / J.grid[0].x;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const float2 g = J.grid[k];
-    const float c0 = blk[k].x - gcur * g.x, c1 = blk[k].y - gcur * g.y;
-    const float v = (c0 * c0 + c1 * c1) * J.pwin[k];
-    const float v3 = v * mult3d;
-    for (int by = y0; by < y1; by++)
-      for (int bx = x0; bx < x1; bx++) {
-        const size_t o = ((size_t)by * J.nox + bx) * n + k;
-        out2d[o] = v;
-        out3d[o] = v3;
-      }
-  }
+  const float v = pattern_term(blk[k], J.grid[k], gcur, J.pwin[k]);
+  const float v3 = v * mult3d;
+  for (int by = y0; by < y1; by++)
+    for (int bx = x0; bx < x1; bx++) {
+      const size_t o = ((size_t)by * J.nox + bx) * n + k;
+      out2d[o] = v;
+      if (out3d) out3d[o] = v3;
+    }
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -159,8 +233,8 @@ hipError_t launch_seam_run(int bw, int bh, const RunBatch& l, hipStream_t s) {
 
 hipError_t launch_pattern(const PatternJob& J, hipStream_t s) {
   int nb = J.nox * J.noy;
-  hipLaunchKernelGGL(k_pattern_sums, dim3((nb + 127) / 128), dim3(128), 0, s, J);
-  hipLaunchKernelGGL(k_pattern_set, dim3(1), dim3(256), 0, s, J);
+  hipLaunchKernelGGL(k_pattern_sums, dim3(nb), dim3(64), 0, s, J);
+  if (J.choice) hipLaunchKernelGGL(k_pattern_set, dim3(1), dim3(256), 0, s, J);
   return hipGetLastError();
 }
 
@@ -168,7 +242,8 @@ hipError_t launch_pattern_regions(const PatternJob& J, int rx, int ry, float* ou
                                   hipStream_t s) {
   if (rx < 1 || ry < 1) return hipErrorInvalidValue;
   const int nq = ((J.nox + rx - 1) / rx) * ((J.noy + ry - 1) / ry);
-  hipLaunchKernelGGL(k_pattern_regions, dim3(nq), dim3(256), 0, s, J, rx, ry, out2d, out3d, mult3d);
+  const int nk = (J.bh * J.outwidth + 255) / 256;
+  hipLaunchKernelGGL(k_pattern_regions, dim3(nq, nk), dim3(256), 0, s, J, rx, ry, out2d, out3d, mult3d);
   return hipGetLastError();
 }
 
