@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "../../include/nf3d.h"
+#include "nf3d_host.h"
 #include "nf3d_internal.h"
 #include "nf3d_mfma.h"
 #include "nf3d_mlp_batch.h"
@@ -131,6 +132,32 @@ T* dev_alloc(size_t count) {
   return static_cast<T*>(p);
 }
 
+uint8_t* pinned_alloc(size_t bytes) {
+  void* p = nullptr;
+  check(hipHostMalloc(&p, std::max<size_t>(bytes, 1), hipHostMallocDefault), "hipHostMalloc");
+  return static_cast<uint8_t*>(p);
+}
+
+// What the runtime knows of p: memory of ordinary allocations (pageable) is
+// Unregistered, hipHostMalloc'd memory Host.
+hipMemoryType memory_type(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return hipMemoryTypeUnregistered;
+  }
+  return a.type;
+}
+
+// Rows between two host buffers.
+void copy_rows(uint8_t* dst, size_t dpitch, const uint8_t* src, size_t spitch, size_t row, int rows) {
+  if (dpitch == row && spitch == row) {
+    memcpy(dst, src, row * rows);
+  } else {
+    for (int y = 0; y < rows; y++) memcpy(dst + y * dpitch, src + y * spitch, row);
+  }
+}
+
 }  // namespace
 
 struct nf3d_engine {
@@ -173,6 +200,13 @@ struct nf3d_engine {
   size_t stage_pitch = 0;
   int stage_next = 0;
   uint8_t* d_dst = nullptr;
+  // pinned staging of the pageable planes of a host-fed frame: an upload
+  // buffer for each plane of one call, and the output's
+  std::vector<uint8_t*> h_up;
+  size_t h_up_used = 0;
+  uint8_t* h_down = nullptr;
+  uint8_t* out_dst = nullptr;  // pageable plane that the frame in flight is copied to (null: none)
+  int out_stride = 0;
   std::mutex mu;
   // Ordering between calls on different streams: the work of the last call
   // ends with done_ev on done_stream, and a call on another stream waits for
@@ -259,6 +293,8 @@ struct nf3d_engine {
     hipFree(d_rsums);
     for (auto* p : d_stage) hipFree(p);
     hipFree(d_dst);
+    for (auto* p : h_up) hipHostFree(p);
+    hipHostFree(h_down);
     for (auto ev : ev_pool) hipEventDestroy(ev);
     if (done_ev) hipEventDestroy(done_ev);
     if (stream) hipStreamDestroy(stream);
@@ -627,9 +663,29 @@ struct nf3d_engine {
     int slot = stage_next;
     stage_next = (stage_next + 1) % (int)d_stage.size();
     stage_frame[slot] = k;
-    check(hipMemcpy2DAsync(d_stage[slot], stage_pitch, fr->data, fr->stride, (size_t)framewidth * pix,
-                           frameheight, hipMemcpyHostToDevice, c.s),
-          "upload");
+    const size_t row = (size_t)framewidth * pix;
+    if (memory_type(fr->data) != hipMemoryTypeUnregistered) {
+      check(hipMemcpy2DAsync(d_stage[slot], stage_pitch, fr->data, fr->stride, row, frameheight, hipMemcpyHostToDevice,
+                             c.s),
+            "upload");
+      return Src{d_stage[slot], (long long)stage_pitch};
+    }
+    // pageable memory: through pinned staging laid out like the device slot,
+    // in chunks that go up while the next one is copied (the runtime's own 2D
+    // copy of pageable rows moved 0.2 GB/s: 11 ms for each plane of a
+    // 1920x1080 frame and way)
+    if (fr->stride < (long long)row) check(hipErrorInvalidPitchValue, "upload");
+    if (h_up_used == h_up.size()) h_up.push_back(pinned_alloc(stage_pitch * frameheight));
+    uint8_t* h = h_up[h_up_used++];
+    const int step = std::max<int>(1, (int)(kUploadChunk / stage_pitch));
+    for (int y = 0; y < frameheight; y += step) {
+      const int rows = std::min(step, frameheight - y);
+      copy_rows(h + (size_t)y * stage_pitch, stage_pitch,
+                static_cast<const uint8_t*>(fr->data) + (size_t)y * fr->stride, fr->stride, row, rows);
+      check(hipMemcpyAsync(d_stage[slot] + (size_t)y * stage_pitch, h + (size_t)y * stage_pitch, stage_pitch * rows,
+                           hipMemcpyHostToDevice, c.s),
+            "upload");
+    }
     return Src{d_stage[slot], (long long)stage_pitch};
   }
 
@@ -1185,21 +1241,69 @@ struct nf3d_engine {
       for (int n = P.b + 1; n < P.first + P.count; n++) run_one(n, P.src, P.src_pitch, P.dst, P.dst_pitch, s);
   }
 
-  void get_frame_host(int n, const nf3d_frame_ref* frames_, int nframes, void* dst, int dst_stride) {
+  static constexpr size_t kUploadChunk = 256 << 10;
+
+  // A host-fed frame: its uploads, filtering and download queued on the
+  // engine's stream ...
+  void frame_begin(int n, const nf3d_frame_ref* frames_, int nframes, void* dst, int dst_stride) {
     Call c{frames_, nframes, false, stream};
     order_before(stream);
-    done_stream = nullptr;  // this call waits for its own work below
+    done_stream = nullptr;  // frame_end waits for the call's work
     std::fill(stage_frame.begin(), stage_frame.end(), -1);
-    size_t dpitch = ((size_t)framewidth * pix + 255) / 256 * 256;
+    h_up_used = 0;
+    out_dst = nullptr;
+    const size_t row = (size_t)Wc * pix, dpitch = ((size_t)framewidth * pix + 255) / 256 * 256;
     if (!d_dst) d_dst = dev_alloc<uint8_t>(dpitch * frameheight);
     run(n, c, d_dst, (long long)dpitch);
-    check(hipMemcpy2DAsync(static_cast<uint8_t*>(dst) + (size_t)tc * dst_stride + (size_t)lc * pix, dst_stride,
-                           d_dst + (size_t)tc * dpitch + (size_t)lc * pix, dpitch, (size_t)Wc * pix, Hc,
-                           hipMemcpyDeviceToHost, stream),
-          "download");
+    uint8_t* from = d_dst + (size_t)tc * dpitch;
+    uint8_t* to = static_cast<uint8_t*>(dst) + (size_t)tc * dst_stride + (size_t)lc * pix;
+    if (memory_type(dst) != hipMemoryTypeUnregistered) {
+      check(hipMemcpy2DAsync(to, dst_stride, from + (size_t)lc * pix, dpitch, row, Hc, hipMemcpyDeviceToHost, stream),
+            "download");
+      return;
+    }
+    if (!dst) check(hipErrorInvalidValue, "download");
+    if (dst_stride < (long long)row) check(hipErrorInvalidPitchValue, "download");
+    if (!h_down) h_down = pinned_alloc(dpitch * frameheight);
+    check(hipMemcpyAsync(h_down, from, dpitch * Hc, hipMemcpyDeviceToHost, stream), "download");
+    out_dst = to;
+    out_stride = dst_stride;
+  }
+  // ... waited for, and its rows handed over.
+  void frame_end() {
     check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    if (!out_dst) return;
+    const size_t dpitch = ((size_t)framewidth * pix + 255) / 256 * 256;
+    copy_rows(out_dst, out_stride, h_down + (size_t)lc * pix, dpitch, (size_t)Wc * pix, Hc);
+    out_dst = nullptr;
   }
 };
+
+int nf3d_engine_frame_begin(nf3d_engine* e, int n, const nf3d_frame_ref* frames, int nframes, void* dst,
+                            int dst_stride, char* err, size_t errlen) {
+  std::unique_lock<std::mutex> lock(e->mu);
+  try {
+    e->last_end = -1;
+    e->frame_begin(n, frames, nframes, dst, dst_stride);
+  } catch (const Failure& f) {
+    (void)hipStreamSynchronize(e->stream);  // the staging buffers are free for the next call
+    copy_err(err, errlen, f.msg);
+    return -1;
+  }
+  lock.release();  // nf3d_engine_frame_end unlocks
+  return 0;
+}
+
+int nf3d_engine_frame_end(nf3d_engine* e, char* err, size_t errlen) {
+  std::unique_lock<std::mutex> lock(e->mu, std::adopt_lock);
+  try {
+    e->frame_end();
+  } catch (const Failure& f) {
+    copy_err(err, errlen, f.msg);
+    return -1;
+  }
+  return 0;
+}
 
 // ---------------------------------------------------------------- C ABI
 extern "C" {
@@ -1260,15 +1364,8 @@ int nf3d_engine_create(const nf3d_params* p, const nf3d_format* fmt, int width, 
 
 int nf3d_engine_get_frame(nf3d_engine* e, int n, const nf3d_frame_ref* frames, int nframes, void* dst,
                           int dst_stride, char* err, size_t errlen) {
-  std::lock_guard<std::mutex> lock(e->mu);
-  try {
-    e->last_end = -1;
-    e->get_frame_host(n, frames, nframes, dst, dst_stride);
-  } catch (const Failure& f) {
-    copy_err(err, errlen, f.msg);
-    return -1;
-  }
-  return 0;
+  if (nf3d_engine_frame_begin(e, n, frames, nframes, dst, dst_stride, err, errlen) != 0) return -1;
+  return nf3d_engine_frame_end(e, err, errlen);
 }
 
 int nf3d_engine_get_frame_device(nf3d_engine* e, int n, const nf3d_frame_ref* frames, int nframes, void* dst,
@@ -1644,15 +1741,8 @@ struct CopyJob {
   int rows;
 };
 // Whether p is page-locked host memory the DMA engines can read directly
-// (hipHostMalloc'd; pageable memory is not known to the runtime).
-bool is_pinned(const void* p) {
-  hipPointerAttribute_t a{};
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return a.type == hipMemoryTypeHost;
-}
+// (hipHostMalloc'd).
+bool is_pinned(const void* p) { return memory_type(p) == hipMemoryTypeHost; }
 
 // Device slots and pinned staging of an engine's host-fed calls, kept from
 // one call to the next and released with the engine (the map itself is never
@@ -1667,11 +1757,7 @@ void run_copies(const std::vector<CopyJob>& jobs) {
   auto work = [&](size_t t) {
     for (size_t j = t; j < jobs.size(); j += nt) {
       const CopyJob& c = jobs[j];
-      if (c.dpitch == c.spitch && c.dpitch == c.row) {
-        memcpy(c.dst, c.src, c.row * c.rows);
-      } else {
-        for (int y = 0; y < c.rows; y++) memcpy(c.dst + y * c.dpitch, c.src + y * c.spitch, c.row);
-      }
+      copy_rows(c.dst, c.dpitch, c.src, c.spitch, c.row, c.rows);
     }
   };
   std::vector<std::thread> th;

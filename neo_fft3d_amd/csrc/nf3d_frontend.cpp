@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/nf3d.h"
+#include "nf3d_host.h"
 
 namespace {
 
@@ -323,7 +324,12 @@ int nf3d_filter_get_frame(nf3d_filter* f, int n, const nf3d_frame_planes* frames
     return -1;
   }
   std::vector<nf3d_frame_ref> refs(nframes);
-  for (int pl = 0; pl < f->fmt.num_planes; pl++) {
+  // every plane is queued (its staging copies overlap the planes before on
+  // the GPU), then each is waited for and copied out
+  nf3d_engine* begun[4];
+  int nbegun = 0;
+  bool ok = true;
+  for (int pl = 0; pl < f->fmt.num_planes && ok; pl++) {
     int w, h;
     f->plane_dims(pl, w, h);
     auto copy_src = [&]() {
@@ -335,12 +341,15 @@ int nf3d_filter_get_frame(nf3d_filter* f, int n, const nf3d_frame_planes* frames
     if (f->process[pl] == 3) {
       if (f->crop) copy_src();  // borders keep the source (src/fft3d.hpp:315-351)
       for (int i = 0; i < nframes; i++) refs[i] = nf3d_frame_ref{frames[i].n, frames[i].data[pl], frames[i].stride[pl]};
-      if (nf3d_engine_get_frame(f->eng[pl], n, refs.data(), nframes, dst[pl], dst_stride[pl], err, errlen) != 0)
-        return -1;
+      ok = nf3d_engine_frame_begin(f->eng[pl], n, refs.data(), nframes, dst[pl], dst_stride[pl], err, errlen) == 0;
+      if (ok) begun[nbegun++] = f->eng[pl];
     } else if (f->process[pl] == 2) {
       copy_src();
     }
   }
+  for (int i = 0; i < nbegun; i++)
+    if (nf3d_engine_frame_end(begun[i], ok ? err : nullptr, ok ? errlen : 0) != 0) ok = false;
+  if (!ok) return -1;
   f->pattern_pending = false;
   return 0;
 }
