@@ -185,7 +185,8 @@ struct nf3d_engine {
   std::vector<char> ring_by_run;  // the slot's spectrum came from the frame-loop kernel
   std::vector<uint64_t> ring_tick;
   uint64_t tick = 0;
-  float2 *d_kal_last = nullptr, *d_kal_covar = nullptr, *d_kal_cproc = nullptr;
+  float2* d_kal_last = nullptr;
+  float* d_kal_sum = nullptr;
   float* d_seam = nullptr;
   int ntx = 0;
   float2* d_spec_tmp = nullptr;
@@ -271,8 +272,7 @@ struct nf3d_engine {
     hipFree(d_grid);
     hipFree(d_ring);
     hipFree(d_kal_last);
-    hipFree(d_kal_covar);
-    hipFree(d_kal_cproc);
+    hipFree(d_kal_sum);
     hipFree(d_seam);
     hipFree(d_seam_run);
     hipFree(d_ones);
@@ -559,13 +559,10 @@ struct nf3d_engine {
     }
     if (ep.bt == 0) {
       d_kal_last = dev_alloc<float2>(spec_elems);
-      d_kal_covar = dev_alloc<float2>(spec_elems);
-      d_kal_cproc = dev_alloc<float2>(spec_elems);
-      std::vector<float2> h(spec_elems, make_float2(0, 0));
-      check(hipMemcpy(d_kal_last, h.data(), spec_elems * sizeof(float2), hipMemcpyHostToDevice), "kalman");
-      std::fill(h.begin(), h.end(), make_float2(sigma2d, sigma2d));
-      check(hipMemcpy(d_kal_covar, h.data(), spec_elems * sizeof(float2), hipMemcpyHostToDevice), "kalman");
-      check(hipMemcpy(d_kal_cproc, h.data(), spec_elems * sizeof(float2), hipMemcpyHostToDevice), "kalman");
+      d_kal_sum = dev_alloc<float>(spec_elems);
+      check(hipMemset(d_kal_last, 0, spec_elems * sizeof(float2)), "kalman");
+      const std::vector<float> h(spec_elems, sigma2d + sigma2d);
+      check(hipMemcpy(d_kal_sum, h.data(), spec_elems * sizeof(float), hipMemcpyHostToDevice), "kalman");
     }
   }
 
@@ -622,8 +619,7 @@ struct nf3d_engine {
     J.use_pattern = ep.pfactor != 0;
     J.use_degrid = ep.degrid != 0;
     J.kal_last = d_kal_last;
-    J.kal_covar = d_kal_covar;
-    J.kal_cproc = d_kal_cproc;
+    J.kal_sum = d_kal_sum;
     J.dft_tab = dft_mode ? dft_tab : nullptr;
     J.dft_sx = dft_sx;
     J.dft_sz = dft_sz;
@@ -1128,6 +1124,7 @@ struct nf3d_engine {
         const int nf = total / nl + (jj >= nl - total % nl ? 1 : 0);
         RunLaunch R{};
         R.J = base_job();
+        R.ntiles = noy * ntx;
         R.J.sigma2 = (float)(P.mode == nf3d::MODE_W3D ? ep.bt : 1) * ep.sigma * ep.sigma / norm;
         R.J.seam = d_seam_run + (size_t)(j & 1) * kRunFrames * seam_frame;
         // learned PSD in d_lpat: predicted from the launch's first frame just
@@ -1145,7 +1142,6 @@ struct nf3d_engine {
         R.m0 = m0;
         R.nframes = nf;
         R.fpw = (P.mode == nf3d::MODE_W3D || P.mode == nf3d::MODE_KALMAN) ? nf : std::min(run_fpw, nf);
-        R.ntiles = noy * ntx;
         P.launches.push_back(R);
         const long long idx = learned_period > 0 ? sp.first / learned_period : -1;
         P.predict.push_back(learned_period <= 0 || (jj == 0 && idx != cur));
@@ -1158,6 +1154,7 @@ struct nf3d_engine {
         if (n >= P.a && n <= P.b) continue;
         RunLaunch R{};
         R.J = base_job();
+        R.ntiles = noy * ntx;
         R.J.sigma2 = ep.sigma * ep.sigma / norm;  // btcur = 1 (src/fft3d_engine.h's window rule)
         R.J.seam = d_seam_run;  // the edge launches run apart from the others on the stream
         if (learned) use_learned(R.J);
@@ -1168,7 +1165,6 @@ struct nf3d_engine {
         R.m0 = n;
         R.nframes = 1;
         R.fpw = 1;
-        R.ntiles = noy * ntx;
         (n < P.a ? P.edges_start : P.edges).push_back(R);
       }
     }
@@ -1200,6 +1196,7 @@ struct nf3d_engine {
         nf3d::RunBatch B{};
         RunLaunch& R = B.job[0];
         R.J = base_job();
+        R.ntiles = noy * ntx;
         R.J.src_pitch = P.src_pitch;
         R.J.dst_pitch = P.dst_pitch;
         for (int k = k0; k < P.a + P.to; k++) R.src[k - k0] = static_cast<const uint8_t*>(P.src[k]);
@@ -1208,7 +1205,6 @@ struct nf3d_engine {
         R.m0 = k0;
         R.nframes = P.a + P.to - k0;
         R.fpw = R.nframes;
-        R.ntiles = noy * ntx;
         R.wg_begin = 0;
         B.njobs = 1;
         B.total_wg = R.ntiles;

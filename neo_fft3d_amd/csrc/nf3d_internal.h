@@ -66,8 +66,7 @@ struct PlaneJob {
   float2* spec_out;          // where this launch's forward spectra are stored (or null)
   const float2* spec_in[5];  // Wiener-3D window, oldest first (on-chip newest: unused)
   float2* kal_last;
-  float2* kal_covar;
-  float2* kal_cproc;
+  float* kal_sum;            // covar + covarProcess (both parts alike)
 };
 
 // One launch: up to three planes of one frame (same block shape).

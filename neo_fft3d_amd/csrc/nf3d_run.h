@@ -802,7 +802,7 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
         constexpr int u = decltype(uu)::value, i = k * CH + u;
         const size_t o = colo + (size_t)i * COLS;
         static_for<0, NQ>([&](auto qq) { b.v[decltype(qq)::value][u] = rq[decltype(qq)::value][o]; });
-        if constexpr (MODE == MODE_KALMAN) b.ks[u] = KalState{J.kal_last[o], J.kal_covar[o], J.kal_cproc[o]};
+        if constexpr (MODE == MODE_KALMAN) b.ks[u] = KalState{J.kal_last[o], J.kal_sum[o]};
       });
     };
     const int tab0 = hh * CR * COLS + cc;  // table element of the lane's first row
@@ -911,8 +911,7 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
             if (col_on) {
               const size_t o = colo + (size_t)i * COLS;
               J.kal_last[o] = st.last;
-              J.kal_covar[o] = st.covar;
-              J.kal_cproc[o] = st.cproc;
+              J.kal_sum[o] = st.sum;
             }
             if constexpr (SHP != SHP_NONE) r = sharpen_s<SHP>(SP, r, T, gfs);
           } else {
