@@ -229,8 +229,7 @@ struct nf3d_engine {
   int run_fpw = 1;              // frames per workgroup, Wiener 2D / sharpen (tuning)
   bool run_frames_from_table = false;  // run_frames came from the tuning table, not the caller
   // 2D transforms: 0 = FFT in registers, 1 = DFT-matrix products on the matrix
-  // cores (32x32 blocks in the frame-loop and the per-frame kernel, 64x64 in the
-  // per-frame kernel)
+  // cores (32x32, 48x48 and 64x64 blocks)
   int dft_mode = 0;
   const void* dft_tab = nullptr;
   float dft_sx = 1.0f, dft_sz = 1.0f;
@@ -1030,6 +1029,20 @@ struct nf3d_engine {
     run(n, c, static_cast<uint8_t*>(dst[n]), dst_pitch);
   }
 
+  // Tiles of a block row in the frame-loop kernel.
+  int run_ntx() const {
+    const int bpw = nf3d::run_blocks_per_wg(ep.bw, ep.bh, dft_mode);
+    return (nox + bpw - 1) / bpw;
+  }
+  // What every frame-loop launch of this engine shares.
+  RunLaunch run_job() const {
+    RunLaunch R{};
+    R.J = base_job();
+    R.J.ntx = run_ntx();
+    R.ntiles = noy * R.J.ntx;
+    return R;
+  }
+
   int shp_kind() const {
     if (ep.sharpen == 0.0f && ep.dehalo == 0.0f) return nf3d::SHP_NONE;
     return ep.dehalo == 0.0f ? nf3d::SHP_SHARPEN : nf3d::SHP_GENERAL;
@@ -1094,10 +1107,11 @@ struct nf3d_engine {
                       (long long)(tc + Hc) * dst_pitch < (1LL << 31) && 4LL * Hc * Wc < (1LL << 31) &&
                       dst_pitch % pix == 0;
     const bool pshow = ep.pfactor != 0 && ep.pshow;
-    // the matrix-core form of 64x64 blocks runs in the per-frame kernel only
-    // (in the frame loop its operands would not fit the registers)
-    const bool mf_tile = dft_mode && ep.bw == 64;
-    P.run = P.a <= P.b && fits && !pshow && !mf_tile && !(P.mode == nf3d::MODE_SHARPEN && P.shp == nf3d::SHP_NONE);
+    // a learned PSD with the matrix-core form of 64x64 blocks is predicted from
+    // each frame itself, in the per-frame path (the frame loop has one
+    // prediction a launch)
+    const bool mf_learned = learned && dft_mode && ep.bw == 64;
+    P.run = P.a <= P.b && fits && !pshow && !mf_learned && !(P.mode == nf3d::MODE_SHARPEN && P.shp == nf3d::SHP_NONE);
     if (!P.run) return P;
     // launches of equal length (within one frame), two halves of seam
     // buffers in turn
@@ -1122,9 +1136,7 @@ struct nf3d_engine {
       const int nl = (total + run_frames - 1) / run_frames;
       for (int jj = 0, m0 = sp.first; jj < nl; jj++, j++) {
         const int nf = total / nl + (jj >= nl - total % nl ? 1 : 0);
-        RunLaunch R{};
-        R.J = base_job();
-        R.ntiles = noy * ntx;
+        RunLaunch R = run_job();
         R.J.sigma2 = (float)(P.mode == nf3d::MODE_W3D ? ep.bt : 1) * ep.sigma * ep.sigma / norm;
         R.J.seam = d_seam_run + (size_t)(j & 1) * kRunFrames * seam_frame;
         // learned PSD in d_lpat: predicted from the launch's first frame just
@@ -1152,9 +1164,7 @@ struct nf3d_engine {
     if (P.mode == nf3d::MODE_W3D) {
       for (int n = first; n < first + count; n++) {
         if (n >= P.a && n <= P.b) continue;
-        RunLaunch R{};
-        R.J = base_job();
-        R.ntiles = noy * ntx;
+        RunLaunch R = run_job();
         R.J.sigma2 = ep.sigma * ep.sigma / norm;  // btcur = 1 (src/fft3d_engine.h's window rule)
         R.J.seam = d_seam_run;  // the edge launches run apart from the others on the stream
         if (learned) use_learned(R.J);
@@ -1195,8 +1205,7 @@ struct nf3d_engine {
       if (k0 < P.a + P.to) {
         nf3d::RunBatch B{};
         RunLaunch& R = B.job[0];
-        R.J = base_job();
-        R.ntiles = noy * ntx;
+        R = run_job();
         R.J.src_pitch = P.src_pitch;
         R.J.dst_pitch = P.dst_pitch;
         for (int k = k0; k < P.a + P.to; k++) R.src[k - k0] = static_cast<const uint8_t*>(P.src[k]);
@@ -1549,7 +1558,7 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
           for (int c = 0; c < B.njobs; c++) evs.push_back(items[members[c0 + c]].engine->timer(timed, 1, s));
           check(nf3d::launch_run(nf3d::MODE_W2D, 0, plans[i].shp, e0->dft_mode, e0->ep.bw, e0->ep.bh, B, s),
                 "frame-loop kernel (clip ends)");
-          check(nf3d::launch_seam_run(e0->ep.bw, e0->ep.bh, B, s), "seam kernel");
+          check(nf3d::launch_seam_run(e0->dft_mode, e0->ep.bw, e0->ep.bh, B, s), "seam kernel");
           for (auto& ev : evs)
             if (ev.second) check(hipEventRecord(ev.second, s), "hipEventRecord");
         }
@@ -1630,7 +1639,7 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
         // launch it takes issue slots the latency-bound k_run needs more
         check(nf3d::launch_run(plans[i].mode, e0->ep.bt, plans[i].shp, e0->dft_mode, e0->ep.bw, e0->ep.bh, B, gs),
               "frame-loop kernel");
-        check(nf3d::launch_seam_run(e0->ep.bw, e0->ep.bh, B, gs), "seam kernel");
+        check(nf3d::launch_seam_run(e0->dft_mode, e0->ep.bw, e0->ep.bh, B, gs), "seam kernel");
         for (auto& ev : evs)
           if (ev.second) check(hipEventRecord(ev.second, gs), "hipEventRecord");
       }

@@ -143,8 +143,9 @@ hipError_t launch_dft_mfma(const void* in, void* out, int nb, int n, int inverse
 // k_run over the batch's jobs; `shp` is a Shp value.  launch_seam_run
 // finishes the seams of their frames (after the k_run, same stream).
 hipError_t launch_run(int mode, int bt, int shp, int mf, int bw, int bh, const RunBatch& b, hipStream_t s);
-hipError_t launch_seam_run(int bw, int bh, const RunBatch& b, hipStream_t s);
+hipError_t launch_seam_run(int mf, int bw, int bh, const RunBatch& b, hipStream_t s);
 bool block_shape_supported(int bw, int bh);
 int tile_blocks_per_wg(int bw, int bh);
+int run_blocks_per_wg(int bw, int bh, int mf);  // of k_run's tiles
 
 }  // namespace nf3d

@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(256) k_pattern_regions(PatternJob J, int rx, i
 #define X(W, H)                                                                                          \
   hipError_t launch_tile_##W##x##H(int mode, int bt, int onchip, int mf, const TileLaunch& l, hipStream_t s); \
   hipError_t launch_run_##W##x##H(int mode, int bt, int shp, int mf, const RunBatch& l, hipStream_t s); \
-  hipError_t launch_seam_run_##W##x##H(const RunBatch& l, hipStream_t s);
+  hipError_t launch_seam_run_##W##x##H(int mf, const RunBatch& l, hipStream_t s);
 NF3D_SHAPES(X)
 #undef X
 
@@ -204,6 +204,11 @@ int tile_blocks_per_wg(int bw, int bh) {
   // TShape<BW,BH,128>::BPW: 128 lanes / max(bw/2+1, bh/2)
   int cols = bw / 2 + 1, pairs = bh / 2;
   return 128 / (cols > pairs ? cols : pairs);
+}
+
+int run_blocks_per_wg(int bw, int bh, int mf) {
+  // RunShape<BW,BH,MF>::BPW
+  return mf && bw == 48 && bh == 48 ? 4 : tile_blocks_per_wg(bw, bh);
 }
 
 bool mfma_dft_supported(int bw, int bh) { return bw == bh && (bw == 32 || bw == 48 || bw == 64); }
@@ -224,8 +229,8 @@ hipError_t launch_run(int mode, int bt, int shp, int mf, int bw, int bh, const R
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_seam_run(int bw, int bh, const RunBatch& l, hipStream_t s) {
-#define X(W, H) if (bw == W && bh == H) return launch_seam_run_##W##x##H(l, s);
+hipError_t launch_seam_run(int mf, int bw, int bh, const RunBatch& l, hipStream_t s) {
+#define X(W, H) if (bw == W && bh == H) return launch_seam_run_##W##x##H(mf, l, s);
   NF3D_SHAPES(X)
 #undef X
   return hipErrorInvalidValue;

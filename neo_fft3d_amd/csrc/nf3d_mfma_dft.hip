@@ -24,7 +24,7 @@ __global__ void __launch_bounds__(256) k_dft_fwd(const float* in, float2* out, i
   const float* X = in + (size_t)blk * N * N;
   const DftIn<N> d = dft_fwd_load<N>([&](int r, int c) { return X[r * N + c]; }, sx, lane);
   float2* o = out + (size_t)blk * N * H;
-  dft_fwd_compute<N>(d, sx, T, lane, [&](int r, int k, float2 z) { o[r * H + k] = z; });
+  dft_fwd_compute<N, false>(d, sx, T, lane, [&](int r, int k, float2 z) { o[r * H + k] = z; });
 }
 
 // Inverse: in [nb][N][N/2+1] float2 -> out [nb][N][N] float (FFTW c2r, unnormalised).
@@ -37,7 +37,7 @@ __global__ void __launch_bounds__(256) k_dft_inv(const float2* in, float* out, i
   const float2* Z = in + (size_t)blk * N * H;
   const DftSpec<N> d = dft_inv_load<N>([&](int r, int k) { return Z[r * H + k]; }, sz, lane);
   float* o = out + (size_t)blk * N * N;
-  dft_inv_compute<N>(d, sz, T, lane, [&](int r, int c0, f4 x) {
+  dft_inv_compute<N, false>(d, sz, T, lane, [&](int r, int c0, f4 x) {
     *reinterpret_cast<float4*>(o + r * N + c0) = make_float4(x[0], x[1], x[2], x[3]);
   });
 }

@@ -6,8 +6,6 @@
 // others between frames.  Per frame the phases are those of k_tile (gather,
 // row r2c, column FFT, spectral pass, column inverse, row c2r, overlap-add);
 // what changes is where the data waits are:
-//   - the pixels of the next frame are loaded into registers before the
-//     current frame's overlap-add, in flight during it and across the barrier;
 //   - the spectral pass runs down each column in chunks of rows: the ring
 //     spectra / Kalman state of chunk k+DR (DR up to 3) and the table rows of
 //     chunk k+1 are loaded while chunk k is computed; the first chunks are
@@ -21,7 +19,7 @@
 // workgroup.  Kalman state likewise stays with its tile.  Seam partials go to
 // a per-frame seam buffer that k_seam_run finishes after the launch.  With MF
 // the row and column transforms are the matrix-core DFT products of
-// nf3d_mfma.h (32x32 blocks).
+// nf3d_mfma.h (32x32, 48x48 and 64x64 blocks).
 #pragma once
 #include "nf3d_tile.h"
 
@@ -61,252 +59,28 @@ __device__ __forceinline__ int batch_job(const RunBatch& B, int wg) {
 // Wavefront of a lane index, as a scalar value.
 __device__ __forceinline__ int wave_of(int t) { return __builtin_amdgcn_readfirstlane(t >> 6); }
 
-template <int I, typename X>
-__device__ __forceinline__ X& pick(X& a, X& b) {
-  if constexpr (I == 0) return a;
-  else return b;
-}
-
-// ------------------------------------------------------------------ gather
-// Rows handled together by the gather's window read-ahead and the
-// overlap-add's LDS reads: a divisor of the rows of a wavefront (8, else 6, 4
-// or 2), so no chunk runs past them.
-template <int RH>
-constexpr int row_chunk() {
-  return RH % 8 == 0 ? 8 : RH % 6 == 0 ? 6 : RH % 4 == 0 ? 4 : 2;
-}
-
-// Work split of the gather and the overlap-add: each wavefront owns RH = BH /
-// (NT / 64) consecutive tile rows, and walks the tile's columns in passes of
-// 64 (lane l: column l + 64 q), so no wavefront runs a pass in which most of
-// its lanes have no column.
-//
-// Raw samples of one lane's columns (up to NQ passes) in this wavefront's RH
-// rows (rowoff: their source row offsets), kept as bits so no use waits on
-// them before the windowing pass.  Every pass is written (zeros past the
-// tile's passes) so no old values stay live around the frame loop.
-template <int PIX, int RH, int NQ>
-__device__ __forceinline__ void gather_issue(const uint8_t* src, const int* rowoff, const int (&sx)[NQ], int npass,
-                                             uint32_t (&raw)[NQ][RH]) {
-  using T = typename std::conditional<PIX == 1, uint8_t, typename std::conditional<PIX == 2, uint16_t, uint32_t>::type>::type;
-  static_for<0, NQ>([&](auto qq) {
-    constexpr int q = decltype(qq)::value;
-    if (q == 0 || q < npass) {  // uniform
-      static_for<0, RH>([&](auto rr) {
-        const T* row = reinterpret_cast<const T*>(src + rowoff[decltype(rr)::value]);
-        raw[q][rr] = (uint32_t)row[sx[q]];
-      });
-    } else {
-      static_for<0, RH>([&](auto rr) { raw[q][rr] = 0u; });
-    }
-  });
-}
-
-// Windowing of the loaded columns into per-block row pairs: the product
-// order of gather_tile ((wx*wy)*p on the outer corners of the edge blocks,
-// (wy*p)*wx on the other windowed columns of the first/last block rows,
-// (wx*p)*wy elsewhere; src/buffer.cpp:137-378).  A column held by one block
-// writes its sample twice to the same place, so no lane branches per row.
-template <int PIX, int BW, int BH, int NT, int SA, int LA, int RH, int NQ>
-__device__ __forceinline__ void gather_window(const PlaneJob& J, float2* stage, const uint32_t (&raw)[NQ][RH],
-                                              const float* winx, const float* winy, int by, int bx0, int nblk,
-                                              int RW, int stepx, int t) {
-  // launch fields as values: one load each, not one per row
-  const int ow = J.ow, oh = J.oh, nox = J.nox, noy = J.noy;
-  const float base = J.base;
-  // lane in the wavefront; its first row (scalar: the row branches below are
-  // uniform per wavefront and compile to scalar branches, not exec masks)
-  const int l = t & 63, r0 = wave_of(t) * RH;
-  constexpr int CW = row_chunk<RH>();  // window rows read ahead together
-  static_for<0, NQ>([&](auto pp) {
-    constexpr int p = decltype(pp)::value;
-    if (p > 0 && p * 64 >= RW) return;  // uniform
-    const int c0 = l + p * 64;
-    const bool cv = c0 < RW;
-    const int c = cv ? c0 : RW - 1;
-    int bA = c / stepx;
-    if (bA >= nblk) bA = nblk - 1;
-    const int jA = c - bA * stepx;
-    const bool hasB = bA >= 1 && jA + stepx < BW;
-    const int bB = hasB ? bA - 1 : bA, jB = hasB ? jA + stepx : jA;
-    auto xinfo = [&](int b, int j, float& wx, int& side, bool& xedge) {
-      side = j < ow ? 1 : (j >= BW - ow ? 2 : 0);
-      wx = winx[j];
-      const int bx = bx0 + b;
-      xedge = (bx == 0 && side == 1) || (bx == nox - 1 && side == 2);
-    };
-    float wxA, wxB;
-    int sA, sB;
-    bool eA, eB;
-    xinfo(bA, jA, wxA, sA, eA);
-    xinfo(bB, jB, wxB, sB, eB);
-    float* dA = reinterpret_cast<float*>(&stage[bA * LA + jA]);
-    float* dB = reinterpret_cast<float*>(&stage[bB * LA + jB]);
-    if (!cv) return;  // tail lanes: nothing to store
-    // per-lane factor of the rows outside the vertical bands: wx on a
-    // windowed column, else 1 ((1*p)*1 = p and (wx*p)*1 = wx*p exactly)
-    const float aA = sA != 0 ? wxA : 1.0f, aB = sB != 0 ? wxB : 1.0f;
-    const bool top_edge = by == 0, bot_edge = by == noy - 1;  // uniform
-    float wyc[CW];  // window values of the current CW rows, read ahead of their use
-    static_for<0, RH>([&](auto rr) {
-      constexpr int u = decltype(rr)::value;
-      const int i = r0 + u;  // tile row (uniform)
-      if constexpr (u % CW == 0) static_for<0, CW>([&](auto uu) { wyc[decltype(uu)::value] = winy[i + decltype(uu)::value]; });
-      float v;
-      if constexpr (PIX == 4) v = __uint_as_float(raw[p][u]);
-      else v = (float)raw[p][u];
-      const float px = v - base;
-      const bool ytop = i < (BH / 2);                // which band, if any (uniform)
-      const bool yw = ytop ? i < oh : i >= BH - oh;  // uniform
-      const int off = (i >> 1) * SA * 2 + (u & 1);   // r0 is even
-      if (!yw) {
-        dA[off] = aA * px;
-        dB[off] = aB * px;
-      } else {
-        const float wy = wyc[u % CW];
-        const bool yedge = ytop ? top_edge : bot_edge;  // uniform
-        auto windowed = [&](float wx, int side, bool xedge) {
-          float a, b;
-          if (!yedge) {
-            a = side != 0 ? wx : wy;
-            b = side != 0 ? wy : 1.0f;
-          } else {
-            a = side != 0 ? (xedge ? wx * wy : wy) : wy;
-            b = side != 0 ? (xedge ? 1.0f : wx) : 1.0f;
-          }
-          return (a * px) * b;
-        };
-        dA[off] = windowed(wxA, sA, eA);
-        dB[off] = windowed(wxB, sB, eB);
-      }
-    });
-  });
-}
-
-// Phase 7 for k_run: overlap-add of the tile in the reference's float order
-// (src/buffer.cpp:381-560), as overlap_tile; lanes compute every row and only
-// the stores are predicated.  The synthesis windows come from LDS: a global
-// load here would wait (vmcnt counts stores too) for every store issued
-// before it.
-template <int PIX, int BW, int BH, int NT, int LSYN, int SYNW>
-__device__ __forceinline__ void overlap_run(const PlaneJob& J, uint8_t* dst, float* seam, const float* syn,
-                                            const float* wsyn, int by, int bx0, int nblk, int RW, int stepx,
-                                            int stepy, int t) {
-  // wsyn: synthesis windows in LDS, [left x (BW) | right x (BW) | top y (BH) |
-  // bottom y (BH)]; one base with computed indices (selecting between table
-  // pointers would put the pointers in scratch memory)
-  constexpr int XL = 0, XR = BW, YL = 2 * BW, YR = 2 * BW + BH;
-  using T = typename std::conditional<PIX == 1, uint8_t, typename std::conditional<PIX == 2, uint16_t, float>::type>::type;
-  const float rounder = PIX == 4 ? 0.0f : 0.5f;
-  // launch fields as values: one load each, not one per row
-  const float fbase = (float)J.obase, norm = J.norm;
-  const int ow = J.ow, oh = J.oh, mirw = J.mirw, mirh = J.mirh, Wc = J.Wc, Hc = J.Hc, maxval = J.maxval;
-  const int interlaced = J.interlaced, half = J.Hc >> 1;
-  const long long dpitch = J.dst_pitch;
-  const int cy0 = by * stepy, cx0 = bx0 * stepx;
-  const size_t P = (size_t)J.seam_plane;
-  uint8_t* dbase = dst + (long long)J.tc * dpitch + (long long)J.lc * sizeof(T);
-  constexpr int NW = NT / 64, RH = BH / NW, NQ = (TShape<BW, BH, 128>::BPW * BW + 63) / 64;
-  constexpr int OC = row_chunk<RH>();  // rows per chunk
-  const int l = t & 63, r0 = wave_of(t) * RH;  // lane in the wavefront; its first row (scalar)
-  static_for<0, NQ>([&](auto pp) {
-    constexpr int p = decltype(pp)::value;
-    if (p > 0 && p * 64 >= RW) return;  // uniform
-    const int xl = l + p * 64;
-    const int x = cx0 + xl - mirw;
-    const bool xin = xl < RW && x >= 0 && x < Wc;
-    // x class: 0 exclusive column, 1 band inside the tile, 2 band shared with
-    // the left tile (this tile holds its right block), 3 band shared with the
-    // right tile (this tile holds its left block)
-    int cls = 0, la = 0, lb = 0;
-    float wa = 0.0f, wb = 1.0f;
-    if (xl < nblk * stepx) {
-      const int bl = xl / stepx, j = xl - bl * stepx;
-      lb = bl * LSYN + j;
-      la = lb;
-      if (j < ow) {
-        wb = wsyn[XL + j];
-        if (bl >= 1) {
-          cls = 1;
-          la = (bl - 1) * LSYN + j + stepx;
-          wa = wsyn[XR + j];
-        } else {
-          cls = 2;
-        }
-      }
-    } else if (xl < RW) {
-      const int jj = xl - nblk * stepx;
-      cls = 3;
-      la = (nblk - 1) * LSYN + stepx + jj;
-      lb = la;
-      wa = wsyn[XR + jj];
-      wb = 0.0f;
-    }
-    const bool own = xin && cls <= 1;   // pixel finished in this tile (body rows)
-    const bool shr = xin && cls >= 2;   // column seam (body rows)
-    // 32-bit element offsets from the uniform plane / seam bases (planes and
-    // seam buffers are < 2^31 elements: checked by the host)
-    const int slot_x = (cls == 3 ? 0 : 1) * (int)P;
-    const int xc = xin ? x : 0;
-    const int pitch_el = (int)(dpitch / (long long)sizeof(T));
-    T* dpl = reinterpret_cast<T*>(dbase);
-    // this wavefront's rows in chunks of OC: the chunk's LDS reads are issued
-    // together, ahead of the per-row (uniform) branches
-#pragma unroll 1
-    for (int i0 = r0; i0 < r0 + RH; i0 += OC) {
-      float h[OC], w[OC];
-      static_for<0, OC>([&](auto uu) {
-        constexpr int u = decltype(uu)::value;
-        const int i = i0 + u;
-        h[u] = syn[la + i * SYNW] * wa + syn[lb + i * SYNW] * wb;
-        w[u] = wsyn[i < oh ? YL + i : (i >= stepy ? YR + i - stepy : YL)];
-      });
-      static_for<0, OC>([&](auto uu) {
-        constexpr int u = decltype(uu)::value;
-        const int i = i0 + u;
-        const int ry = cy0 + i - mirh;
-        if (ry >= 0 && ry < Hc) {  // not a padding row (uniform)
-          // output row (interlaced fields stacked, second field bottom-up)
-          const int yo = !interlaced ? ry : (ry < half ? 2 * ry : Hc - 1 - 2 * (ry - half));
-          const int so = yo * Wc + xc;
-          if (i >= oh && i < stepy) {  // rows of this block row only (uniform)
-            const float v = h[u] * norm + rounder + fbase;
-            T q;
-            if constexpr (PIX == 4) {
-              const float o = v < 0.0f ? 0.0f : v;
-              q = o > 1.0f ? 1.0f : o;
-            } else {
-              int qi = (int)v;
-              qi = qi < 0 ? 0 : qi;
-              q = (T)(qi > maxval ? maxval : qi);
-            }
-            if (own) dpl[(unsigned)(yo * pitch_el + xc)] = q;
-            if (shr) seam[(unsigned)(slot_x + so)] = h[u];  // slot 0 = left block's part, slot 1 = right's
-          } else {
-            const bool ytop = i < oh;
-            // row seam: slot 0 = upper block row's part, slot 1 = lower's
-            // (times its window); corner: A upper-left, B upper-right, C
-            // lower-left, D lower-right
-            const int slot = cls <= 1 ? (ytop ? 1 : 0) : (ytop ? (cls == 3 ? 2 : 3) : (cls == 3 ? 0 : 1));
-            const float val = cls <= 1 ? h[u] * (w[u] * norm) : h[u];
-            if (xin) seam[(unsigned)(slot * (int)P + so)] = val;
-          }
-        }
-      });
-    }
-  });
-}
+// A workgroup's tile: a lane pair per spectral column and per row pair of
+// each block, so that BPW blocks fill the 256 lanes.  The matrix-core form of
+// 48x48 blocks takes four, one per wavefront: a fifth costs its transforms a
+// second round in which three wavefronts wait (tiles are only a split of the
+// work: every pixel's sums keep their order).
+template <int BW, int BH, bool MF>
+struct RunShape : TShape<BW, BH, 128, (MF && BW == 48 && BH == 48) ? 4 : 0> {};
 
 // ------------------------------------------- gather / overlap-add by column
-// 256-lane tiles: lane (block b, column j) reads block b's column j of every
-// row straight from the plane (reflect-101 addressing) and writes it,
-// windowed, into the block's row pairs -- no per-pass column mapping, one
-// store per sample.  The window product is (p * wx) * wy for every sample:
-// the same value as the region-by-region order of gather_window up to one
-// rounding (the parity bar is against the FP64 product).
-template <int PIX, int BW, int BH, int SA, int LA>
+// Lane (block b, column j) reads block b's column j of every row straight
+// from the plane (reflect-101 addressing) and writes it, windowed, into the
+// block's row pairs -- no per-pass column mapping, one store per sample.
+// The window product is (p * wx) * wy for every sample: the value of the
+// region-by-region order of gather_tile (wx or wy is exactly 1 outside its
+// bands) except in the bands at the plane's top and bottom edge, where that
+// order multiplies by wy first, or by wx * wy at the corners; one rounding
+// apart (the parity bar is against the FP64 product).  EDGE: that order there
+// too (the matrix-core form keeps it; only tiles of the first and last block
+// row pay for the selection).
+template <int PIX, int BW, int BH, int SA, int LA, bool EDGE>
 __device__ __forceinline__ void gather_cols(const PlaneJob& J, float2* stage, const uint8_t* src, const int* rowoff,
-                                            const float* winx, const float* winy, int bx0, int nblk, int stepx,
+                                            const float* winx, const float* winy, int by, int bx0, int nblk, int stepx,
                                             int t) {
   using T = typename std::conditional<PIX == 1, uint8_t, typename std::conditional<PIX == 2, uint16_t, float>::type>::type;
   const int b = t / BW, j = t - b * BW;
@@ -322,17 +96,34 @@ __device__ __forceinline__ void gather_cols(const PlaneJob& J, float2* stage, co
     v[i] = *reinterpret_cast<const T*>(src + (unsigned)(rowoff[i] + sxb));
   });
   float* d = reinterpret_cast<float*>(&stage[b * LA + j]);
-  static_for<0, BH>([&](auto ii) {
-    constexpr int i = decltype(ii)::value;
-    const float px = (float)v[i] - base;
-    d[(i >> 1) * SA * 2 + (i & 1)] = (px * wx) * winy[i];
-  });
+  if constexpr (EDGE) {
+    const int top = by == 0 ? J.oh : 0, bot = by == J.noy - 1 ? BH - J.oh : BH;  // uniform
+    const int bx = bx0 + b;
+    const bool xedge = (bx == 0 && j < J.ow) || (bx == J.nox - 1 && j >= BW - J.ow);
+    static_for<0, BH>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const float px = (float)v[i] - base, wy = winy[i];
+      const bool yedge = i < top || i >= bot;
+      const float f0 = yedge ? (xedge ? wx * wy : wy) : wx;
+      const float f1 = yedge ? (xedge ? 1.0f : wx) : wy;
+      d[(i >> 1) * SA * 2 + (i & 1)] = (px * f0) * f1;
+    });
+  } else {
+    static_for<0, BH>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      const float px = (float)v[i] - base;
+      d[(i >> 1) * SA * 2 + (i & 1)] = (px * wx) * winy[i];
+    });
+  }
 }
 
 // Overlap-add with one lane per tile column, down all BH rows of the tile's
 // block row: the column's block(s) and synthesis weights are worked out once
 // per frame, then each row is one or two LDS reads and its store -- the
-// reference's float order of overlap_run (src/buffer.cpp:381-560).
+// reference's float order (src/buffer.cpp:381-560).  The synthesis windows
+// come from LDS, [left x (BW) | right x (BW) | top y (BH) | bottom y (BH)]: a
+// global load here would wait (vmcnt counts stores too) for every store
+// issued before it.
 template <int PIX, int BW, int BH, int LSYN, int SYNW>
 __device__ __forceinline__ void overlap_cols(const PlaneJob& J, uint8_t* dst, float* seam, const float* syn,
                                              const float* wsyn, int by, int bx0, int nblk, int RW, int stepx,
@@ -520,42 +311,41 @@ __device__ __forceinline__ void split_combine_inv(float2 (&c)[BH / 2], int h, fl
 // mask keeps its old value in the other lanes, which would hold it live around
 // the frame loop.
 //
-// MF: the 2D transforms as DFT-matrix products on the matrix cores (32x32
-// and 48x48 blocks, nf3d_mfma.h), a wavefront per block in turn, in place of the row
-// and column FFTs; the spectral pass is unchanged.
+// Each spectral column has a lane pair, which runs the spectral pass over half
+// of the column's rows each.
 //
-// NT = 256 (FFT form): the tile of the 128-lane geometry (BPW blocks) with
-// twice the lanes.  Gather and overlap-add split the tile's rows over four
-// wavefronts; the row transforms use the first BPW * BH/2 lanes (the other
-// wavefronts skip them); each spectral column has a lane pair, which splits
-// its transform in two half-length transforms (split_combine_*) and runs the
-// spectral pass over half of the column's rows each.
+// FFT form: gather and overlap-add by column; the row transforms use the first
+// BPW * BH/2 * 2 lanes (the other wavefronts skip them); a lane pair splits a
+// row pair's or a column's transform in two half-length transforms
+// (split_combine_*).
 //
-// Waves per SIMD the register budget is cut for (256 lanes: LDS allows three
-// workgroups per CU at 48x48): three, or two for the variants whose spectral
-// pass holds more per element (four or five frames, the dehalo factor, the
-// Kalman state with a sharpen pass, 64-row columns), which would otherwise
-// spill.  128 lanes (the matrix-core form): two at 32x32, one at 48x48 (256
-// VGPRs and the AGPRs, no spills).
-template <int BH, int NT, int MODE, int BT, int SHP, bool MF>
+// MF: the 2D transforms as DFT-matrix products on the matrix cores (32x32,
+// 48x48 and 64x64 blocks, nf3d_mfma.h), a wavefront per block in turn, in
+// place of the row and column FFTs.  With two lanes a column and rolled tile
+// loops it takes 128 / 155 / 188 registers (32 / 48 / 64, bt = 3), so two to
+// four wavefronts share a SIMD: 48/16 on 3840x2160 4:2:0, 8 frames, 3480 us
+// at one wavefront per SIMD with 424 registers, 1800 us now.
+//
+// Waves per SIMD the register budget is cut for (LDS allows three workgroups
+// per CU at 48x48): three, or two for the variants whose spectral pass holds
+// more per element (four or five frames, the dehalo factor, the Kalman state
+// with a sharpen pass, 64-row columns), which would otherwise spill.
+template <int BH, int MODE, int BT, int SHP>
 constexpr int run_waves_per_simd() {
-  if constexpr (MF && BH >= 48) return 1;
-  else if constexpr (NT != 256) return 2;
-  else if constexpr (BH >= 64 || (MODE == MODE_W3D && (BT >= 4 || SHP == SHP_GENERAL)) ||
-                     (MODE == MODE_KALMAN && SHP != SHP_NONE))
+  if constexpr (BH >= 64 || (MODE == MODE_W3D && (BT >= 4 || SHP == SHP_GENERAL)) ||
+                (MODE == MODE_KALMAN && SHP != SHP_NONE))
     return 2;
   else return 3;
 }
 
 template <int BW, int BH, int NT, int MODE, int BT, int SHP, bool MF = false>
-__global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP, MF>())) k_run(RunBatch B_arg) {
+__global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>())) k_run(RunBatch B_arg) {
   const RunBatch& B0 = kernarg_batch(B_arg);
   const int jb = batch_job(B0, blockIdx.x);
   const RunLaunch& L0 = B0.job[jb];
-  using S = TShape<BW, BH, 128>;
-  constexpr bool SPLIT = NT == 256;
-  static_assert(NT == 128 || (NT == 256 && !MF), "256 lanes: the FFT form");
-  constexpr int CR = SPLIT ? BH / 2 : BH;  // spectral rows per column lane
+  using S = RunShape<BW, BH, MF>;
+  static_assert(NT == 256, "a lane pair per spectral column of BPW blocks");
+  constexpr int CR = BH / 2;  // spectral rows per column lane
   constexpr int COLS = S::COLS, PAIRS = S::PAIRS, BPW = S::BPW, SR = S::SR, LSPEC = S::LSPEC;
   constexpr int SYNW = S::SYNW, LSYN = S::LSYN, SA = S::SA, LA = S::LA;
   constexpr int FROM = MODE == MODE_W3D ? -(BT / 2) : 0;
@@ -568,9 +358,8 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
   // (m0 + i) % BT -- the Wiener-3D window frames a range starts with, so
   // every spectrum in the ring comes from this kernel's arithmetic
   // chunks of ring rows in flight ahead of the one being computed
-  // (256 lanes: half the rows per lane and a register budget of 168 for
-  // three wavefronts per SIMD)
-  constexpr int DR = MODE == MODE_W3D ? (SPLIT ? (NQ <= 2 ? 2 : 1) : (NQ <= 2 ? 3 : NQ == 3 ? 2 : 1)) : 1;
+  // (a register budget of 168 for three wavefronts per SIMD)
+  constexpr int DR = MODE == MODE_W3D && NQ <= 2 ? 2 : 1;
   using RBuf = RingBuf<MODE, NQ, CH>;
   using TBuf = TabBuf<SHP, CH>;
   __shared__ __align__(16) unsigned char smem[S::BYTES];
@@ -595,11 +384,6 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
   const int nblk = min(BPW, L0.J.nox - bx0);
   const int stepx = BW - L0.J.ow, stepy = BH - L0.J.oh;
   const int RW = (nblk - 1) * stepx + BW;
-  // gather / overlap-add split: RH rows per wavefront, up to GQ column passes
-  constexpr int RH = BH / (NT / 64), GQ = (BPW * BW + 63) / 64;
-  static_assert(NT % 64 == 0 && BH % (NT / 64) == 0 && RH % 2 == 0, "row split");
-  const int npass = (RW + 63) >> 6;
-
   {
     const PlaneJob& J = L0.J;
     const int t = threadIdx.x;
@@ -619,23 +403,6 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
   }
   __syncthreads();
 
-  // pixels of a frame's on-chip transform (this wavefront's rows), loaded
-  // one frame ahead
-  uint32_t raw[GQ][RH];
-  auto issue = [&](const PlaneJob& J, const uint8_t* src, const int* ro, int t) {
-    const int l = t & 63;
-    int sx[GQ];
-    static_for<0, GQ>([&](auto qq) {
-      constexpr int q = decltype(qq)::value;
-      sx[q] = reflect101(bx0 * stepx + min(l + 64 * q, RW - 1) - J.mirw, J.Wc) + J.lc;
-    });
-    const int* rw = ro + wave_of(t) * RH;
-    if (J.pix == 1) gather_issue<1, RH, GQ>(src, rw, sx, npass, raw);
-    else if (J.pix == 2) gather_issue<2, RH, GQ>(src, rw, sx, npass, raw);
-    else gather_issue<4, RH, GQ>(src, rw, sx, npass, raw);
-  };
-  if constexpr (!SPLIT) issue(L0.J, L0.src[i0], rowoff, (int)threadIdx.x);
-
 #pragma unroll 1
   for (int fi = i0; fi < i1; fi++) {
     // The lane index, the launch record and the LDS tables are reached
@@ -653,21 +420,19 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
     const int* ro = rowoff + zo;
     const int m = L.m0 + fi;
     const int pix = J.pix;
-    // column lanes: one per column, or a pair (SPLIT: hh = half, rows
-    // hh * CR .. hh * CR + CR - 1 of the spectrum after the forward transform)
-    const int cl = SPLIT ? (t >> 1) : t;
-    const int hh = SPLIT ? (t & 1) : 0;
+    // column lanes: a pair per column (half hh: rows hh * CR .. hh * CR + CR - 1
+    // of the spectrum after the forward transform)
+    const int cl = t >> 1, hh = t & 1;
     const float sg = hh ? -1.0f : 1.0f;
     const int cbr = cl / COLS, cc = cl - cbr * COLS;
     const bool col_on = cbr < nblk;
     const int cb = col_on ? cbr : nblk - 1;
-    // row lanes: one per row pair, or a pair of lanes (SPLIT, half hh)
-    const int rl = SPLIT ? (t >> 1) : t;
-    const int rbr = rl / PAIRS, rp = rl - rbr * PAIRS;
+    // row lanes: a pair per row pair
+    const int rbr = cl / PAIRS, rp = cl - rbr * PAIRS;
     const bool row_on = rbr < nblk;
     const int rb = row_on ? rbr : nblk - 1;
     // wavefronts with no row pair of the tile skip the row transforms
-    const bool row_wave = wave_of(t) * 64 < BPW * PAIRS * (SPLIT ? 2 : 1);
+    const bool row_wave = wave_of(t) * 64 < BPW * PAIRS * 2;
     const size_t tile_spec0 = (size_t)(by * J.nox + bx0) * (BH * COLS);
     // element (hh * CR, cc) of this lane's column: its first spectral row
     const size_t colo = tile_spec0 + (size_t)cb * (BH * COLS) + (size_t)(hh * CR) * COLS + cc;
@@ -679,16 +444,16 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
     const float grid0 = J.grid[0].x;
     const SpecParams SP(J);
 
-    // ---- 1. window the loaded pixels into per-block row pairs
-    if constexpr (SPLIT) {
-      const uint8_t* fsrc = L.src[fi];
-      if (pix == 1) gather_cols<1, BW, BH, SA, LA>(J, stage, fsrc, ro, wx, wy, bx0, nblk, stepx, t);
-      else if (pix == 2) gather_cols<2, BW, BH, SA, LA>(J, stage, fsrc, ro, wx, wy, bx0, nblk, stepx, t);
-      else gather_cols<4, BW, BH, SA, LA>(J, stage, fsrc, ro, wx, wy, bx0, nblk, stepx, t);
+    // ---- 1. windowed pixels into per-block row pairs
+    const uint8_t* fsrc = L.src[fi];
+    if (MF && (by == 0 || by == J.noy - 1)) {
+      if (pix == 1) gather_cols<1, BW, BH, SA, LA, MF>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
+      else if (pix == 2) gather_cols<2, BW, BH, SA, LA, MF>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
+      else gather_cols<4, BW, BH, SA, LA, MF>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
     } else {
-      if (pix == 1) gather_window<1, BW, BH, NT, SA, LA, RH, GQ>(J, stage, raw, wx, wy, by, bx0, nblk, RW, stepx, t);
-      else if (pix == 2) gather_window<2, BW, BH, NT, SA, LA, RH, GQ>(J, stage, raw, wx, wy, by, bx0, nblk, RW, stepx, t);
-      else gather_window<4, BW, BH, NT, SA, LA, RH, GQ>(J, stage, raw, wx, wy, by, bx0, nblk, RW, stepx, t);
+      if (pix == 1) gather_cols<1, BW, BH, SA, LA, false>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
+      else if (pix == 2) gather_cols<2, BW, BH, SA, LA, false>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
+      else gather_cols<4, BW, BH, SA, LA, false>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
     }
     __syncthreads();
     if constexpr (MF) {
@@ -705,22 +470,22 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
       const float sx = J.dft_sx;
 #pragma unroll 1
       for (int q = 0; q < MB; q++) {
-        const int b = nblk - 1 - (q * NW + wave);  // uniform in the wavefront
-        DftIn<BW> din;
-        if (b >= 0)
-          din = dft_fwd_load<BW>(
-              [&](int r, int c) {
-                const float2 v = stage[b * LA + (r >> 1) * SA + c];
-                return (r & 1) ? v.y : v.x;
-              },
-              sx, lane);
+        // (a wavefront past the tile's blocks loads block 0's place and does
+        // not use it: operands loaded under a branch would keep their old
+        // values alive around the loops)
+        const int b = nblk - 1 - (q * NW + wave), bl = max(b, 0);  // uniform in the wavefront
+        const DftIn<BW> din = dft_fwd_load<BW>(
+            [&](int r, int c) {
+              return reinterpret_cast<const float*>(stage)[2 * (bl * LA + (r >> 1) * SA + c) + (r & 1)];
+            },
+            sx, lane);
         __syncthreads();  // the round's stages read
         if (b >= 0)
-          dft_fwd_compute<BW>(din, sx, T, lane, [&](int r, int k, float2 zz) { spec[b * LSPEC + r * SR + k] = zz; });
+          dft_fwd_compute<BW, true>(din, sx, T, lane, [&](int r, int k, float2 zz) { spec[b * LSPEC + r * SR + k] = zz; });
       }
     } else if (!row_wave) {
       __syncthreads();  // gather stage dead; spectral layout from here
-    } else if constexpr (SPLIT) {
+    } else {
       // ---- 2. row r2c, a lane pair per two real rows packed as one complex
       // row Z: the BW-point transform as two BW/2-point transforms of its even
       // and odd columns combined across the pair (lane 0: Z[k], lane 1:
@@ -749,40 +514,20 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
           dst[SR + q] = make_float2((a.y + b.y) * 0.5f, (b.x - a.x) * 0.5f);
         }
       });
-    } else {
-      // ---- 2. row r2c, two real rows per lane
-      float2 z[BW];
-      static_for<0, BW>([&](auto j) { z[j] = stage[rb * LA + rp * SA + decltype(j)::value]; });
-      __syncthreads();  // gather stage dead; spectral layout from here
-      fft<BW, -1>(z);
-      if (row_on) {
-        float2* dst = spec + rb * LSPEC + 2 * rp * SR;
-        static_for<0, COLS>([&](auto kk) {
-          constexpr int k = decltype(kk)::value;
-          constexpr int km = (BW - k) % BW;
-          const float2 a = z[k], b = z[km];
-          dst[k] = make_float2((a.x + b.x) * 0.5f, (a.y - b.y) * 0.5f);
-          dst[SR + k] = make_float2((a.y + b.y) * 0.5f, (b.x - a.x) * 0.5f);
-        });
-      }
     }
     __syncthreads();
 
+    // row of the tile's spectral layout that the lane's value j has in LDS: the
+    // rows of its half, or (FFT form) even rows on lane 0, odd rows on lane 1
+    auto col_row = [=](auto j) { return MF ? hh * CR + decltype(j)::value : 2 * decltype(j)::value + hh; };
     if constexpr (MODE == MODE_FWD) {
       // ---- 3. forward column transforms to the ring, then the next frame
       float2 fc[CR];
-      if constexpr (SPLIT) {
-        static_for<0, CR>([&](auto j) { fc[j] = spec[cb * LSPEC + (2 * decltype(j)::value + hh) * SR + cc]; });
-      } else {
-        static_for<0, CR>([&](auto i) { fc[i] = spec[cb * LSPEC + decltype(i)::value * SR + cc]; });
-      }
+      static_for<0, CR>([&](auto j) { fc[j] = spec[cb * LSPEC + col_row(j) * SR + cc]; });
       __syncthreads();  // spectra read: the next frame's gather may write the stage
-      if constexpr (!SPLIT) issue(J, L.src[min(fi + 1, i1 - 1)], ro, t);
-      if constexpr (SPLIT) {
+      if constexpr (!MF) {
         fft<CR, -1>(fc);
         split_combine_fwd<BH>(fc, hh, sg);
-      } else if constexpr (!MF) {
-        fft<BH, -1>(fc);
       }
       if (col_on) {
         float2* out = L.ring + (size_t)(m % BT) * L.spec_elems + colo;
@@ -837,14 +582,10 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
     float2 col[CR];
     static_for<0, (DR < NCH ? DR : NCH)>([&](auto kc) { load_ring(kc, rbuf[decltype(kc)::value]); });
     load_tab(std::integral_constant<int, 0>{}, tbuf[0]);
-    if constexpr (SPLIT) {
-      // even rows on lane 0, odd rows on lane 1
-      static_for<0, CR>([&](auto j) { col[j] = spec[cb * LSPEC + (2 * decltype(j)::value + hh) * SR + cc]; });
+    static_for<0, CR>([&](auto j) { col[j] = spec[cb * LSPEC + col_row(j) * SR + cc]; });
+    if constexpr (!MF) {
       fft<CR, -1>(col);
       split_combine_fwd<BH>(col, hh, sg);
-    } else {
-      static_for<0, BH>([&](auto i) { col[i] = spec[cb * LSPEC + decltype(i)::value * SR + cc]; });
-      if constexpr (!MF) fft<BH, -1>(col);
     }
     if constexpr (MODE == MODE_W3D) {
       if (col_on) {
@@ -933,17 +674,12 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
       });
     }
     // ---- 5. column inverse FFT, back to LDS for the row c2r
-    if constexpr (SPLIT) {
+    if constexpr (!MF) {
       split_combine_inv<BH>(col, hh, sg);
       fft<CR, +1>(col);
-      if (col_on) {
-        static_for<0, CR>([&](auto j) { spec[cb * LSPEC + (2 * decltype(j)::value + hh) * SR + cc] = col[j]; });
-      }
-    } else {
-      if constexpr (!MF) fft<BH, +1>(col);
-      if (col_on) {
-        static_for<0, BH>([&](auto i) { spec[cb * LSPEC + decltype(i)::value * SR + cc] = col[i]; });
-      }
+    }
+    if (col_on) {
+      static_for<0, CR>([&](auto j) { spec[cb * LSPEC + col_row(j) * SR + cc] = col[j]; });
     }
     __syncthreads();
     if constexpr (MF) {
@@ -959,12 +695,11 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
       const float sz = J.dft_sz;
 #pragma unroll 1
       for (int q = 0; q < MB; q++) {
-        const int b = q * NW + wave;  // uniform in the wavefront
-        DftSpec<BW> dsp;
-        if (b < nblk) dsp = dft_inv_load<BW>([&](int r, int k) { return spec[b * LSPEC + r * SR + k]; }, sz, lane);
+        const int b = q * NW + wave, bl = min(b, nblk - 1);  // uniform in the wavefront
+        const DftSpec<BW> dsp = dft_inv_load<BW>([&](int r, int k) { return spec[bl * LSPEC + r * SR + k]; }, sz, lane);
         __syncthreads();  // the round's spectra read
         if (b < nblk)
-          dft_inv_compute<BW>(dsp, sz, T, lane, [&](int r, int c0, f4 x) {
+          dft_inv_compute<BW, true>(dsp, sz, T, lane, [&](int r, int c0, f4 x) {
             float* d = syn + b * LSYN + r * SYNW + c0;
             d[0] = x[0];
             d[1] = x[1];
@@ -974,7 +709,7 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
       }
     } else if (!row_wave) {
       __syncthreads();  // spectral layout dead; synthesised rows next
-    } else if constexpr (SPLIT) {
+    } else {
       // ---- 6. row c2r, a lane pair per two rows: each lane builds the packed
       // spectrum z (Hermitian rows packed, DC and Nyquist imaginary parts
       // dropped) and reduces it to its half-length inverse transform's input
@@ -1020,49 +755,15 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, NT, MODE, BT, SHP,
           d0[SYNW + 2 * decltype(j)::value] = z[j].y;
         });
       }
-    } else {
-      // ---- 6. row c2r (Hermitian rows packed in pairs; DC and Nyquist imag dropped)
-      float2 z[BW];
-      const float2* src = spec + rb * LSPEC + 2 * rp * SR;
-      static_for<0, COLS>([&](auto kk) {
-        constexpr int k = decltype(kk)::value;
-        float2 a = src[k], b = src[SR + k];
-        if constexpr (k == 0 || 2 * k == BW) {
-          a.y = 0.0f;
-          b.y = 0.0f;
-        }
-        z[k] = make_float2(a.x - b.y, a.y + b.x);
-        if constexpr (k != 0 && 2 * k != BW) z[BW - k] = make_float2(a.x + b.y, b.x - a.y);
-      });
-      __syncthreads();  // spectral layout dead; synthesised rows next
-      fft<BW, +1>(z);
-      if (row_on) {
-        float* d0 = syn + rb * LSYN + 2 * rp * SYNW;
-        static_for<0, BW>([&](auto j) {
-          d0[decltype(j)::value] = z[j].x;
-          d0[SYNW + decltype(j)::value] = z[j].y;
-        });
-      }
     }
     __syncthreads();
-    // ---- the next frame's pixels, in flight during the overlap-add and
-    // across the barrier (the registers of the row transforms are dead here;
-    // the last iteration reloads its own frame: an unconditional load keeps
-    // the old values from living through the iteration)
-    if constexpr (!SPLIT) issue(J, L.src[min(fi + 1, i1 - 1)], ro, t);
     // ---- 7. overlap-add inside the tile; seam partials to this frame's seam buffer
     uint8_t* dst = L.dst[fi];
     float* seam = J.seam + (size_t)fi * 4 * (size_t)J.seam_plane;
     const float* ws = wsyn + zo;
-    if constexpr (SPLIT) {
-      if (pix == 1) overlap_cols<1, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-      else if (pix == 2) overlap_cols<2, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-      else overlap_cols<4, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-    } else {
-      if (pix == 1) overlap_run<1, BW, BH, NT, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-      else if (pix == 2) overlap_run<2, BW, BH, NT, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-      else overlap_run<4, BW, BH, NT, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-    }
+    if (pix == 1) overlap_cols<1, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
+    else if (pix == 2) overlap_cols<2, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
+    else overlap_cols<4, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
     __syncthreads();  // syn read; the next frame's gather writes the stage
   }
 }
@@ -1084,11 +785,10 @@ __device__ __forceinline__ int div_small(int n, int d, float inv) {
 // row: both band partials are loaded unconditionally (8 pixels per lane in
 // flight), the corner partials where a vertical seam crosses.  Other rows
 // finish only the columns of the vertical seams between tiles.
-template <int BW, int BH, int NT>
+template <int BW, int BH, int BPW>
 __global__ void __launch_bounds__(256) k_seam_run(RunBatch B_arg) {
   const RunLaunch& L = kernarg_batch(B_arg).job[blockIdx.z];
   const PlaneJob& J = L.J;
-  constexpr int BPW = TShape<BW, BH, NT>::BPW;
   const int yo = blockIdx.x;
   const int fi = blockIdx.y;
   if (yo >= J.Hc || fi >= L.nframes) return;
@@ -1150,7 +850,7 @@ __global__ void __launch_bounds__(256) k_seam_run(RunBatch B_arg) {
 
 template <int BW, int BH, bool MF>
 hipError_t launch_run_modes(int mode, int bt, int shp, const RunBatch& L, hipStream_t s) {
-  constexpr int NT = MF ? 128 : 256;
+  constexpr int NT = 256;
   dim3 grid(L.total_wg), block(NT);
 #define NF3D_RUN(M, B, H) hipLaunchKernelGGL((k_run<BW, BH, NT, M, B, H, MF>), grid, block, 0, s, L)
 #define NF3D_RUN_SHP(M, B)                                   \
@@ -1193,7 +893,7 @@ hipError_t launch_run_modes(int mode, int bt, int shp, const RunBatch& L, hipStr
   return hipGetLastError();
 }
 
-// mf: the matrix-core DFT form (32x32 and 48x48 blocks).
+// mf: the matrix-core DFT form (32x32, 48x48 and 64x64 blocks).
 template <int BW, int BH>
 hipError_t launch_run_shape(int mode, int bt, int shp, int mf, const RunBatch& L, hipStream_t s) {
   if (L.njobs < 1 || L.njobs > RUN_MAX_JOBS) return hipErrorInvalidValue;
@@ -1206,19 +906,24 @@ hipError_t launch_run_shape(int mode, int bt, int shp, int mf, const RunBatch& L
   }
   if (wg != L.total_wg) return hipErrorInvalidValue;
   if (mf) {
-    // 64x64 blocks in the matrix-core form go through the per-frame kernel
-    // (in the frame loop their operands would exceed the register file)
-    if constexpr (BW == BH && (BW == 32 || BW == 48)) return launch_run_modes<BW, BH, true>(mode, bt, shp, L, s);
+    if constexpr (BW == BH && (BW == 32 || BW == 48 || BW == 64)) return launch_run_modes<BW, BH, true>(mode, bt, shp, L, s);
     else return hipErrorInvalidValue;
   }
   return launch_run_modes<BW, BH, false>(mode, bt, shp, L, s);
 }
 
 template <int BW, int BH>
-hipError_t launch_seam_run_shape(const RunBatch& L, hipStream_t s) {
+hipError_t launch_seam_run_shape(int mf, const RunBatch& L, hipStream_t s) {
   if (L.njobs < 1 || L.njobs > RUN_MAX_JOBS || L.max_frames < 1 || L.max_frames > RUN_MAX_FRAMES) return hipErrorInvalidValue;
   dim3 sgrid(L.max_hc, L.max_frames, L.njobs);
-  hipLaunchKernelGGL((k_seam_run<BW, BH, 128>), sgrid, dim3(256), 0, s, L);
+  constexpr int BPW = RunShape<BW, BH, false>::BPW, BPW_MF = RunShape<BW, BH, true>::BPW;
+  if constexpr (BPW_MF != BPW) {
+    if (mf) {
+      hipLaunchKernelGGL((k_seam_run<BW, BH, BPW_MF>), sgrid, dim3(256), 0, s, L);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((k_seam_run<BW, BH, BPW>), sgrid, dim3(256), 0, s, L);
   return hipGetLastError();
 }
 

@@ -293,12 +293,13 @@ __device__ __forceinline__ const TileLaunch& kernarg_launch(const TileLaunch& ar
 }
 
 // ------------------------------------------------------------------ shapes
-template <int BW, int BH, int NT>
+// BLOCKS: blocks of a tile (0: as many as the lanes hold)
+template <int BW, int BH, int NT, int BLOCKS = 0>
 struct TShape {
   static constexpr int PAIRS = BH / 2;
   static constexpr int COLS = BW / 2 + 1;
   static constexpr int TPB = COLS > PAIRS ? COLS : PAIRS;
-  static constexpr int BPW = NT / TPB;
+  static constexpr int BPW = BLOCKS ? BLOCKS : NT / TPB;
   static constexpr int SR = COLS;                  // spectral row stride (float2)
   static constexpr int LSPEC = BH * SR;            // float2 per block
   static constexpr int SYNW = BW + 1;              // synthesised row stride (float)
@@ -544,7 +545,7 @@ __global__ void __launch_bounds__(NT) k_tile(TileLaunch L_arg) {
               sx, lane);
         __syncthreads();  // the round's stages read
         if (b >= 0)
-          dft_fwd_compute<BW>(din, sx, T, lane, [&](int r, int k, float2 zz) { spec[b * LSPEC + r * SR + k] = zz; });
+          dft_fwd_compute<BW, true>(din, sx, T, lane, [&](int r, int k, float2 zz) { spec[b * LSPEC + r * SR + k] = zz; });
       }
     } else {
       // ---- 2. row r2c, two real rows per lane
@@ -703,7 +704,7 @@ __global__ void __launch_bounds__(NT) k_tile(TileLaunch L_arg) {
         if (b < nblk) dsp = dft_inv_load<BW>([&](int r, int k) { return spec[b * LSPEC + r * SR + k]; }, sz, lane);
         __syncthreads();  // the round's spectra read
         if (b < nblk)
-          dft_inv_compute<BW>(dsp, sz, T, lane, [&](int r, int c0, f4 x) {
+          dft_inv_compute<BW, true>(dsp, sz, T, lane, [&](int r, int c0, f4 x) {
             float* d = syn + b * LSYN + r * SYNW + c0;
             d[0] = x[0];
             d[1] = x[1];
