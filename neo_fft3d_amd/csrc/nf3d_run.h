@@ -255,52 +255,69 @@ struct TabBuf {
   float wdh[SHP == SHP_GENERAL ? CH : 1];
 };
 
-// ------------------------------------------------------- split column FFT
-// The value of the other lane of a lane pair (lanes 2c, 2c+1): a DPP
-// quad permutation [1,0,3,2], one VALU instruction per 32-bit value.
-__device__ __forceinline__ float pair_swap(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float2 pair_swap(float2 v) { return make_float2(pair_swap(v.x), pair_swap(v.y)); }
+// ------------------------------------------------------------- split FFTs
+// A transform of N points is split over a pair of lanes l and l + 32 of a
+// wavefront (h = 0, 1): two transforms of N/2 points, of the even values on
+// lane l and of the odd ones on lane l + 32, and one radix-2 step.  The swap
+// below gives each lane both operands of half of that step's butterflies, so
+// no lane computes a butterfly's half that the other lane also computes (with
+// a full exchange, both lanes twiddled and half of the results were thrown
+// away: 10 instructions a value instead of 6).
 
-// Forward BH-point column DFT split over a lane pair: lane h holds the
-// BH/2-point DFT of the column's rows h, h+2, h+4, ... (E for h = 0, O for
-// h = 1).  X[k] = E[k] + w^k O[k] and X[k + BH/2] = E[k] - w^k O[k]
-// (w = exp(-2 pi i / BH)): lane 1 twiddles, the pair exchanges, lane 0 keeps
-// X[k] and lane 1 X[k + BH/2], k < BH/2.  `sg` is +1 on lane 0, -1 on lane 1
-// (fma by +-1 is an exact add / subtract).
-template <int BH>
-__device__ __forceinline__ void split_combine_fwd(float2 (&c)[BH / 2], int h, float sg) {
-  static_for<0, BH / 2>([&](auto kk) {
+// Exchanges a of the upper 32 lanes with b of the lower 32.
+__device__ __forceinline__ void half_swap(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void half_swap(float2& a, float2& b) {
+  half_swap(a.x, b.x);
+  half_swap(a.y, b.y);
+}
+// The other lane's value of the pair.
+__device__ __forceinline__ float2 half_other(float2 v, int h) {
+  float2 a = v, b = v;
+  half_swap(a, b);  // a: the lower lanes' value, b: the upper lanes'
+  return h ? a : b;
+}
+
+// Forward radix-2 step: in, c[k] = E[k] (lane 0) / O[k] (lane 1), k < N/2; out,
+// X[k] = E[k] + w^k O[k] and X[k + N/2] = E[k] - w^k O[k], w = exp(-2 pi i / N):
+// lane h holds X[h N/4 + i] in c[i] and X[N/2 + h N/4 + i] in c[N/4 + i],
+// i < N/4.  (w^(k + N/4) = -i w^k: the same product, turned, on lane 1.)
+template <int N>
+__device__ __forceinline__ void split_combine_fwd(float2 (&c)[N / 2], int h) {
+  static_for<0, N / 4>([&](auto kk) {
     constexpr int k = decltype(kk)::value;
-    float2 v = c[k];
+    float2 e = c[k], o = c[k + N / 4];
+    half_swap(e, o);
     if constexpr (k != 0) {
-      constexpr float wr = (float)ct::cos2pi(k, BH), wi = (float)(-ct::sin2pi(k, BH));
-      const float2 tw = cmul(v, wr, wi);
-      v = h ? tw : v;
+      constexpr float wr = (float)ct::cos2pi(k, N), wi = (float)(-ct::sin2pi(k, N));
+      o = cmul(o, wr, wi);
     }
-    const float2 p = pair_swap(v);
-    c[k] = make_float2(__builtin_fmaf(sg, v.x, p.x), __builtin_fmaf(sg, v.y, p.y));
+    o = h ? make_float2(o.y, -o.x) : o;
+    c[k] = cadd(e, o);
+    c[k + N / 4] = csub(e, o);
   });
 }
 
-// Inverse of the above (unnormalised, FFTW c2r convention): lane 0 holds
-// X[k], lane 1 X[k + BH/2]; the even output rows are the BH/2-point inverse
-// DFT of X[k] + X[k + BH/2], the odd rows that of w^-k (X[k] - X[k + BH/2]).
-// Lane h ends with the inputs of its BH/2-point inverse transform.
-template <int BH>
-__device__ __forceinline__ void split_combine_inv(float2 (&c)[BH / 2], int h, float sg) {
-  static_for<0, BH / 2>([&](auto kk) {
+// Inverse of the above (unnormalised, FFTW c2r convention), X in lane h as
+// split_combine_fwd leaves it: the even values come from the N/2-point
+// inverse transform of X[k] + X[k + N/2], the odd ones from that of
+// w^-k (X[k] - X[k + N/2]); lane h ends with the inputs of its half.
+template <int N>
+__device__ __forceinline__ void split_combine_inv(float2 (&c)[N / 2], int h) {
+  static_for<0, N / 4>([&](auto kk) {
     constexpr int k = decltype(kk)::value;
-    const float2 v = c[k];
-    const float2 p = pair_swap(v);
-    float2 d = make_float2(__builtin_fmaf(sg, v.x, p.x), __builtin_fmaf(sg, v.y, p.y));
+    float2 s = cadd(c[k], c[k + N / 4]), d = csub(c[k], c[k + N / 4]);
     if constexpr (k != 0) {
-      constexpr float wr = (float)ct::cos2pi(k, BH), wi = (float)ct::sin2pi(k, BH);
-      const float2 tw = cmul(d, wr, wi);
-      d = h ? tw : d;
+      constexpr float wr = (float)ct::cos2pi(k, N), wi = (float)ct::sin2pi(k, N);
+      d = cmul(d, wr, wi);
     }
-    c[k] = d;
+    d = h ? make_float2(-d.y, d.x) : d;
+    half_swap(s, d);
+    c[k] = s;
+    c[k + N / 4] = d;
   });
 }
 
@@ -389,7 +406,8 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     const int t = threadIdx.x;
     for (int i = t; i < BW; i += NT) winx[i] = J.wanx[i];
     for (int i = t; i < BH; i += NT) {
-      winy[i] = J.wany[i];
+      // (the FFT form's row transforms take halved samples: exact)
+      winy[i] = MF ? J.wany[i] : 0.5f * J.wany[i];
       rowoff[i] = (int)((long long)(cover_to_src_row(J, by * stepy + i) + J.tc) * J.src_pitch);
     }
     for (int i = t; i < J.ow; i += NT) {
@@ -420,10 +438,10 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     const int* ro = rowoff + zo;
     const int m = L.m0 + fi;
     const int pix = J.pix;
-    // column lanes: a pair per column (half hh: rows hh * CR .. hh * CR + CR - 1
-    // of the spectrum after the forward transform)
-    const int cl = t >> 1, hh = t & 1;
-    const float sg = hh ? -1.0f : 1.0f;
+    // column lanes: a pair (l, l + 32) per column, half hh: rows hh * CR/2 + i
+    // and BH/2 + hh * CR/2 + i, i < CR/2, of the spectrum after the forward
+    // transform (value j of the lane: row hh * CR/2 + col_row(j))
+    const int cl = (t >> 6) * 32 + (t & 31), hh = (t >> 5) & 1;
     const int cbr = cl / COLS, cc = cl - cbr * COLS;
     const bool col_on = cbr < nblk;
     const int cb = col_on ? cbr : nblk - 1;
@@ -432,14 +450,13 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     const bool row_on = rbr < nblk;
     const int rb = row_on ? rbr : nblk - 1;
     // wavefronts with no row pair of the tile skip the row transforms
-    const bool row_wave = wave_of(t) * 64 < BPW * PAIRS * 2;
+    const bool row_wave = wave_of(t) * 32 < BPW * PAIRS;
     const size_t tile_spec0 = (size_t)(by * J.nox + bx0) * (BH * COLS);
-    // element (hh * CR, cc) of this lane's column: its first spectral row
-    const size_t colo = tile_spec0 + (size_t)cb * (BH * COLS) + (size_t)(hh * CR) * COLS + cc;
+    // element (hh * CR/2, cc) of this lane's column: its first spectral row
+    const size_t colo = tile_spec0 + (size_t)cb * (BH * COLS) + (size_t)(hh * (CR / 2)) * COLS + cc;
     // the pattern: one for the plane, or this block's (learned PSD)
     const float* pat = J.use_pattern ? (MODE == MODE_W3D ? J.pattern3d : J.pattern2d) +
-                                           (J.pattern_per_block ? colo - (size_t)(hh * CR) * COLS - cc : 0) +
-                                           (size_t)(hh * CR) * COLS
+                                           (J.pattern_per_block ? colo - cc : (size_t)(hh * (CR / 2)) * COLS)
                                      : nullptr;
     const float grid0 = J.grid[0].x;
     const SpecParams SP(J);
@@ -487,51 +504,64 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
       __syncthreads();  // gather stage dead; spectral layout from here
     } else {
       // ---- 2. row r2c, a lane pair per two real rows packed as one complex
-      // row Z: the BW-point transform as two BW/2-point transforms of its even
-      // and odd columns combined across the pair (lane 0: Z[k], lane 1:
-      // Z[k + BW/2]); after an exchange each lane finishes half of the output
-      // columns k (lane 0: 0..BW/4, lane 1: BW/4+1..BW/2) from Z[k] and
-      // Z[BW - k].
-      constexpr int HW = BW / 2, K0 = HW / 2 + 1;
+      // row (samples halved by the window): its BW-point transform Z split
+      // over the pair, then the rows' spectra (Z[k] + conj Z[BW-k]) and
+      // (Z[k] - conj Z[BW-k]) / i.  With Q = BW/4, lane 0 holds Z[i] and
+      // Z[2Q + i], lane 1 Z[Q + i] and Z[3Q + i] (P[i] and R[i]); two values
+      // i = j, j + Q/2 of both are swapped so that lane 0 has all four of j
+      // and lane 1 all four of j + Q/2, each the columns i and Q + i.
+      constexpr int HW = BW / 2, Q = BW / 4;
       float2 z[HW];
       static_for<0, HW>([&](auto j) { z[j] = stage[rb * LA + rp * SA + 2 * decltype(j)::value + hh]; });
       __syncthreads();  // gather stage dead; spectral layout from here
       fft<HW, -1>(z);
-      split_combine_fwd<BW>(z, hh, sg);
-      float2 o[HW];
-      static_for<0, HW>([&](auto j) { o[j] = pair_swap(z[j]); });
-      // lane 0: low half Z[0..HW) = z, high half = o; lane 1 the other way round
-      float2* dst = spec + rb * LSPEC + 2 * rp * SR + hh * K0;
-      static_for<0, K0>([&](auto qq) {
-        constexpr int q = decltype(qq)::value;
-        constexpr int k1 = K0 + q;  // lane 1's column
-        const float2 a0 = z[q], b0 = q == 0 ? z[0] : o[(HW - q) % HW];
-        const float2 a1 = k1 < HW ? o[k1 < HW ? k1 : 0] : z[0];
-        const float2 b1 = z[k1 <= HW ? HW - k1 : 0];
-        const float2 a = hh ? a1 : a0, b = hh ? b1 : b0;
-        if (row_on && (hh == 0 || k1 <= HW)) {
-          dst[q] = make_float2((a.x + b.x) * 0.5f, (a.y - b.y) * 0.5f);
-          dst[SR + q] = make_float2((a.y + b.y) * 0.5f, (b.x - a.x) * 0.5f);
-        }
+      split_combine_fwd<BW>(z, hh);
+      float2* row = spec + rb * LSPEC + 2 * rp * SR;
+      auto put = [&](float2* d, float2 a, float2 b) {  // columns from Z[k] and Z[BW - k]
+        d[0] = make_float2(a.x + b.x, a.y - b.y);
+        d[SR] = make_float2(a.y + b.y, b.x - a.x);
+      };
+      // (every lane exchanges; lanes without a row pair of the tile store nothing)
+      static_for<1, Q / 2>([&](auto jj) {
+        constexpr int j = decltype(jj)::value;
+        half_swap(z[j], z[j + Q / 2]);              // lane 0: P[j] of both lanes; lane 1: P[j + Q/2] of both
+        half_swap(z[HW - j], z[HW - j - Q / 2]);    // ... R[Q - j], R[Q - j - Q/2]
       });
+      const float2 other = half_other(z[Q + Q / 2], hh);
+      if (row_on) {
+        static_for<1, Q / 2>([&](auto jj) {
+          constexpr int j = decltype(jj)::value;
+          float2* d = row + hh * (Q / 2) + j;
+          put(d, z[j], z[HW - j - Q / 2]);
+          put(d + Q, z[j + Q / 2], z[HW - j]);
+        });
+        put(row + Q / 2 + hh * Q, z[Q / 2], other);       // i = Q/2: P[i] with the other lane's R[Q - i]
+        put(row + hh * Q, z[0], hh ? z[Q] : z[0]);        // column 0 / Q
+        if (hh == 0) put(row + HW, z[Q], z[Q]);           // column BW/2
+      }
     }
     __syncthreads();
 
-    // row of the tile's spectral layout that the lane's value j has in LDS: the
-    // rows of its half, or (FFT form) even rows on lane 0, odd rows on lane 1
-    auto col_row = [=](auto j) { return MF ? hh * CR + decltype(j)::value : 2 * decltype(j)::value + hh; };
+    // row (past hh * CR/2) of the lane's value j in the spectrum ...
+    auto col_row = [](auto j) { return decltype(j)::value + (decltype(j)::value >= CR / 2 ? CR / 2 : 0); };
+    // ... and the LDS row it is read from and goes back to: that row, or (FFT
+    // form) the transforms' inputs and outputs, even rows on lane 0, odd on lane 1
+    auto lds_row = [=](auto j) {
+      return MF ? hh * (CR / 2) + decltype(j)::value + (decltype(j)::value >= CR / 2 ? CR / 2 : 0)
+                : 2 * decltype(j)::value + hh;
+    };
     if constexpr (MODE == MODE_FWD) {
       // ---- 3. forward column transforms to the ring, then the next frame
       float2 fc[CR];
-      static_for<0, CR>([&](auto j) { fc[j] = spec[cb * LSPEC + col_row(j) * SR + cc]; });
+      static_for<0, CR>([&](auto j) { fc[j] = spec[cb * LSPEC + lds_row(j) * SR + cc]; });
       __syncthreads();  // spectra read: the next frame's gather may write the stage
       if constexpr (!MF) {
         fft<CR, -1>(fc);
-        split_combine_fwd<BH>(fc, hh, sg);
+        split_combine_fwd<BH>(fc, hh);
       }
       if (col_on) {
         float2* out = L.ring + (size_t)(m % BT) * L.spec_elems + colo;
-        static_for<0, CR>([&](auto i) { out[decltype(i)::value * COLS] = fc[i]; });
+        static_for<0, CR>([&](auto i) { out[col_row(i) * COLS] = fc[i]; });
       }
       continue;
     }
@@ -545,23 +575,26 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
       constexpr int k = decltype(kc)::value;
       static_for<0, CH>([&](auto uu) {
         constexpr int u = decltype(uu)::value, i = k * CH + u;
-        const size_t o = colo + (size_t)i * COLS;
+        const size_t o = colo + (size_t)col_row(std::integral_constant<int, i>{}) * COLS;
         static_for<0, NQ>([&](auto qq) { b.v[decltype(qq)::value][u] = rq[decltype(qq)::value][o]; });
         if constexpr (MODE == MODE_KALMAN) b.ks[u] = KalState{J.kal_last[o], J.kal_sum[o]};
       });
     };
-    const int tab0 = hh * CR * COLS + cc;  // table element of the lane's first row
+    const int tab0 = hh * (CR / 2) * COLS + cc;  // table element of the lane's first row
     auto load_tab = [&](auto kc, TBuf& b) {
       constexpr int k = decltype(kc)::value;
       static_for<0, CH>([&](auto uu) {
         constexpr int u = decltype(uu)::value, i = k * CH + u;
-        const int kk = i * COLS + tab0;
+        const int kk = col_row(std::integral_constant<int, i>{}) * COLS + tab0;
         b.g[u] = J.grid[kk];
         if constexpr (SHP != SHP_NONE) b.wsh[u] = J.wsharpen[kk];
         if constexpr (SHP == SHP_GENERAL) b.wdh[u] = J.wdehalo[kk];
       });
       if (pat) {
-        static_for<0, CH>([&](auto uu) { b.sig[decltype(uu)::value] = pat[(k * CH + decltype(uu)::value) * COLS + cc]; });
+        static_for<0, CH>([&](auto uu) {
+          constexpr int i = k * CH + decltype(uu)::value;
+          b.sig[decltype(uu)::value] = pat[col_row(std::integral_constant<int, i>{}) * COLS + cc];
+        });
       } else {
         static_for<0, CH>([&](auto uu) { b.sig[decltype(uu)::value] = J.sigma2; });
       }
@@ -582,15 +615,15 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     float2 col[CR];
     static_for<0, (DR < NCH ? DR : NCH)>([&](auto kc) { load_ring(kc, rbuf[decltype(kc)::value]); });
     load_tab(std::integral_constant<int, 0>{}, tbuf[0]);
-    static_for<0, CR>([&](auto j) { col[j] = spec[cb * LSPEC + col_row(j) * SR + cc]; });
+    static_for<0, CR>([&](auto j) { col[j] = spec[cb * LSPEC + lds_row(j) * SR + cc]; });
     if constexpr (!MF) {
       fft<CR, -1>(col);
-      split_combine_fwd<BH>(col, hh, sg);
+      split_combine_fwd<BH>(col, hh);
     }
     if constexpr (MODE == MODE_W3D) {
       if (col_on) {
         float2* out = L.ring + (size_t)((m + TO) % BT) * L.spec_elems + colo;
-        static_for<0, CR>([&](auto i) { out[decltype(i)::value * COLS] = col[i]; });
+        static_for<0, CR>([&](auto i) { out[col_row(i) * COLS] = col[i]; });
       }
     }
     // ---- 4a. per-block degrid fractions from the input DC and from the
@@ -650,7 +683,7 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
             KalState st = b.ks[u];
             r = kalman_elem(SP, col[i], T, st);
             if (col_on) {
-              const size_t o = colo + (size_t)i * COLS;
+              const size_t o = colo + (size_t)col_row(std::integral_constant<int, i>{}) * COLS;
               J.kal_last[o] = st.last;
               J.kal_sum[o] = st.sum;
             }
@@ -675,11 +708,11 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     }
     // ---- 5. column inverse FFT, back to LDS for the row c2r
     if constexpr (!MF) {
-      split_combine_inv<BH>(col, hh, sg);
+      split_combine_inv<BH>(col, hh);
       fft<CR, +1>(col);
     }
     if (col_on) {
-      static_for<0, CR>([&](auto j) { spec[cb * LSPEC + col_row(j) * SR + cc] = col[j]; });
+      static_for<0, CR>([&](auto j) { spec[cb * LSPEC + lds_row(j) * SR + cc] = col[j]; });
     }
     __syncthreads();
     if constexpr (MF) {
@@ -710,42 +743,28 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     } else if (!row_wave) {
       __syncthreads();  // spectral layout dead; synthesised rows next
     } else {
-      // ---- 6. row c2r, a lane pair per two rows: each lane builds the packed
-      // spectrum z (Hermitian rows packed, DC and Nyquist imaginary parts
-      // dropped) and reduces it to its half-length inverse transform's input
-      // (split_combine_inv: lane 0 z[k] + z[k + BW/2], lane 1
-      // w^-k (z[k] - z[k + BW/2])); lane h ends with output columns 2j + h.
-      constexpr int HW = BW / 2;
-      const float2* src = spec + rb * LSPEC + 2 * rp * SR;
-      auto zcol = [&](auto kk) {  // z[k] (k <= HW) from column k
-        constexpr int k = decltype(kk)::value;
-        float2 a = src[k], b = src[SR + k];
-        if constexpr (k == 0 || k == HW) {
-          a.y = 0.0f;
-          b.y = 0.0f;
-        }
-        return make_float2(a.x - b.y, a.y + b.x);
-      };
-      auto zmirror = [&](auto kk) {  // z[BW - k] (0 < k < HW) from column k
-        constexpr int k = decltype(kk)::value;
-        const float2 a = src[k], b = src[SR + k];
-        return make_float2(a.x + b.y, b.x - a.y);
-      };
+      // ---- 6. row c2r, a lane pair per two rows: lane h builds Z[k] and
+      // Z[k + BW/2], k = h BW/4 + i, of the packed spectrum from columns k and
+      // BW/2 - k of both rows (DC and Nyquist imaginary parts dropped) and the
+      // pair reduces them to its half-length inverse transforms' inputs; lane
+      // h ends with output columns 2j + h.
+      constexpr int HW = BW / 2, Q = BW / 4;
+      const float2* lo = spec + rb * LSPEC + 2 * rp * SR + hh * Q;         // column k = lo[i]
+      const float2* hi = spec + rb * LSPEC + 2 * rp * SR + HW - hh * Q;    // column BW/2 - k = hi[-i]
       float2 z[HW];
-      static_for<0, HW>([&](auto kk) {
-        constexpr int k = decltype(kk)::value;
-        const float2 zl = zcol(kk);
-        float2 zu;
-        if constexpr (k == 0) zu = zcol(std::integral_constant<int, HW>{});
-        else zu = zmirror(std::integral_constant<int, HW - k>{});
-        float2 d = make_float2(__builtin_fmaf(sg, zu.x, zl.x), __builtin_fmaf(sg, zu.y, zl.y));
-        if constexpr (k != 0) {
-          constexpr float wr = (float)ct::cos2pi(k, BW), wi = (float)ct::sin2pi(k, BW);
-          const float2 tw = cmul(d, wr, wi);
-          d = hh ? tw : d;
+      static_for<0, Q>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        float2 a = lo[i], b = lo[SR + i], c = hi[-i], d = hi[SR - i];
+        if constexpr (i == 0) {  // lane 0: columns 0 and BW/2
+          a.y = hh ? a.y : 0.0f;
+          b.y = hh ? b.y : 0.0f;
+          c.y = hh ? c.y : 0.0f;
+          d.y = hh ? d.y : 0.0f;
         }
-        z[k] = d;
+        z[i] = make_float2(a.x - b.y, a.y + b.x);
+        z[Q + i] = make_float2(c.x + d.y, d.x - c.y);
       });
+      split_combine_inv<BW>(z, hh);
       __syncthreads();  // spectral layout dead; synthesised rows next
       fft<HW, +1>(z);
       if (row_on) {
