@@ -69,137 +69,219 @@ struct RunShape : TShape<BW, BH, 128, (MF && BW == 48 && BH == 48) ? 4 : 0> {};
 
 // ------------------------------------------- gather / overlap-add by column
 // Lane (block b, column j) reads block b's column j of every row straight
-// from the plane (reflect-101 addressing) and writes it, windowed, into the
-// block's row pairs -- no per-pass column mapping, one store per sample.
-// The window product is (p * wx) * wy for every sample: the value of the
+// from the plane (reflect-101 addressing), kept as bits so that no use waits
+// on a load before the windowing.  Lanes past the tile's blocks load its last
+// block's.
+template <int BW, int BH>
+__device__ __forceinline__ void gather_load(const PlaneJob& J, uint32_t (&raw)[BH], const uint8_t* src,
+                                            const int* rowoff, int bx0, int nblk, int stepx, int t) {
+  const int tb = t / BW, b = min(tb, nblk - 1), j = t - tb * BW;
+  const int sx = reflect101((bx0 + b) * stepx + j - J.mirw, J.Wc) + J.lc;
+  // 32-bit byte offsets from the uniform plane base: one add per sample
+  // (rows are < 2^31 bytes from the base: checked by the host)
+  auto load = [&](auto* as) {
+    using T = typename std::remove_pointer<decltype(as)>::type;
+    const int sxb = sx * (int)sizeof(T);
+    static_for<0, BH>([&](auto ii) {
+      raw[ii] = *reinterpret_cast<const T*>(src + (unsigned)(rowoff[decltype(ii)::value] + sxb));
+    });
+  };
+  if (J.pix == 1) load((uint8_t*)nullptr);  // (uniform)
+  else if (J.pix == 2) load((uint16_t*)nullptr);
+  else load((uint32_t*)nullptr);
+}
+
+// The loaded samples, windowed, into the block's row pairs.  The window
+// product is (p * wx) * wy for every sample: the value of the
 // region-by-region order of gather_tile (wx or wy is exactly 1 outside its
 // bands) except in the bands at the plane's top and bottom edge, where that
 // order multiplies by wy first, or by wx * wy at the corners; one rounding
 // apart (the parity bar is against the FP64 product).  EDGE: that order there
 // too (the matrix-core form keeps it; only tiles of the first and last block
 // row pay for the selection).
-template <int PIX, int BW, int BH, int SA, int LA, bool EDGE>
-__device__ __forceinline__ void gather_cols(const PlaneJob& J, float2* stage, const uint8_t* src, const int* rowoff,
-                                            const float* winx, const float* winy, int by, int bx0, int nblk, int stepx,
-                                            int t) {
-  using T = typename std::conditional<PIX == 1, uint8_t, typename std::conditional<PIX == 2, uint16_t, float>::type>::type;
+template <int BW, int BH, int SA, int LA, bool EDGE>
+__device__ __forceinline__ void gather_window(const PlaneJob& J, float2* stage, const uint32_t (&raw)[BH],
+                                              const float* winx, const float* winy, int by, int bx0, int nblk, int t) {
   const int b = t / BW, j = t - b * BW;
   if (b >= nblk) return;  // lanes past the tile's blocks
-  const int sx = reflect101((bx0 + b) * stepx + j - J.mirw, J.Wc) + J.lc;
-  const float wx = winx[j], base = J.base;
-  // 32-bit byte offsets from the uniform plane base: one add per sample
-  // (rows are < 2^31 bytes from the base: checked by the host)
-  const int sxb = sx * (int)sizeof(T);
-  T v[BH];
-  static_for<0, BH>([&](auto ii) {
-    constexpr int i = decltype(ii)::value;
-    v[i] = *reinterpret_cast<const T*>(src + (unsigned)(rowoff[i] + sxb));
-  });
+  const float wx = winx[j];
   float* d = reinterpret_cast<float*>(&stage[b * LA + j]);
-  if constexpr (EDGE) {
-    const int top = by == 0 ? J.oh : 0, bot = by == J.noy - 1 ? BH - J.oh : BH;  // uniform
-    const int bx = bx0 + b;
-    const bool xedge = (bx == 0 && j < J.ow) || (bx == J.nox - 1 && j >= BW - J.ow);
-    static_for<0, BH>([&](auto ii) {
-      constexpr int i = decltype(ii)::value;
-      const float px = (float)v[i] - base, wy = winy[i];
-      const bool yedge = i < top || i >= bot;
-      const float f0 = yedge ? (xedge ? wx * wy : wy) : wx;
-      const float f1 = yedge ? (xedge ? 1.0f : wx) : wy;
-      d[(i >> 1) * SA * 2 + (i & 1)] = (px * f0) * f1;
-    });
-  } else {
-    static_for<0, BH>([&](auto ii) {
-      constexpr int i = decltype(ii)::value;
-      const float px = (float)v[i] - base;
-      d[(i >> 1) * SA * 2 + (i & 1)] = (px * wx) * winy[i];
-    });
-  }
+  auto window = [&](auto value) {  // (value: the sample less the centring)
+    if constexpr (EDGE) {
+      const int top = by == 0 ? J.oh : 0, bot = by == J.noy - 1 ? BH - J.oh : BH;  // uniform
+      const int bx = bx0 + b;
+      const bool xedge = (bx == 0 && j < J.ow) || (bx == J.nox - 1 && j >= BW - J.ow);
+      static_for<0, BH>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        const float px = value(raw[i]), wy = winy[i];
+        const bool yedge = i < top || i >= bot;
+        const float f0 = yedge ? (xedge ? wx * wy : wy) : wx;
+        const float f1 = yedge ? (xedge ? 1.0f : wx) : wy;
+        d[(i >> 1) * SA * 2 + (i & 1)] = (px * f0) * f1;
+      });
+    } else {
+      static_for<0, BH>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        const float px = value(raw[i]);
+        d[(i >> 1) * SA * 2 + (i & 1)] = (px * wx) * winy[i];
+      });
+    }
+  };
+  const float base = J.base;
+  if (J.pix == 4) window([](uint32_t r) { return __uint_as_float(r); });  // (uniform; float planes are not centred)
+  else if (base == 0.0f) window([](uint32_t r) { return (float)r; });
+  else window([=](uint32_t r) { return (float)r - base; });
 }
 
-// Overlap-add with one lane per tile column, down all BH rows of the tile's
-// block row: the column's block(s) and synthesis weights are worked out once
-// per frame, then each row is one or two LDS reads and its store -- the
-// reference's float order (src/buffer.cpp:381-560).  The synthesis windows
-// come from LDS, [left x (BW) | right x (BW) | top y (BH) | bottom y (BH)]: a
+// n / d for 0 <= n < 2^22 and 1 <= d <= 64 (inv = 1/d rounded): the float
+// quotient is within one of the exact one, and one correction each way
+// makes it exact.
+__device__ __forceinline__ int div_small(int n, int d, float inv) {
+  int q = (int)((float)n * inv);
+  const int r = n - q * d;
+  q += r >= d ? 1 : 0;
+  q -= r < 0 ? 1 : 0;
+  return q;
+}
+
+// Overlap-add of the tile rows [r0, r1) (uniform) in NQ tile columns per lane,
+// xl + 64 q, in the reference's float order (src/buffer.cpp:381-560): the
+// columns' block(s), synthesis weights and offsets are worked out once; then
+// the rows of the upper band, of this block row alone and of the lower band
+// each in a loop without a condition per row, the LDS reads of RC rows in
+// every column together.  A loop's last rows may repeat its last row (the same
+// value to the same place).  wsyn: [left x (BW) | right x (BW) | top y (BH) |
+// bottom y (BH)], the y windows times norm; rowdst: element offset of each
+// tile row in a seam plane (x) and in the destination (y).  Both in LDS: a
 // global load here would wait (vmcnt counts stores too) for every store
 // issued before it.
-template <int PIX, int BW, int BH, int LSYN, int SYNW>
-__device__ __forceinline__ void overlap_cols(const PlaneJob& J, uint8_t* dst, float* seam, const float* syn,
-                                             const float* wsyn, int by, int bx0, int nblk, int RW, int stepx,
-                                             int stepy, int t) {
-  constexpr int XL = 0, XR = BW, YL = 2 * BW, YR = 2 * BW + BH;
+template <int PIX, int BW, int BH, int LSYN, int SYNW, int NQ>
+__device__ __forceinline__ void overlap_rows(const PlaneJob& J, uint8_t* dst, float* seam, const float* syn,
+                                             const float* wsyn, const int2* rowdst, int by, int bx0, int nblk, int RW,
+                                             int stepx, int stepy, int xl, int r0, int r1) {
+  constexpr int XL = 0, XR = BW, YL = 2 * BW, YR = 2 * BW + BH, RC = 4;
   using T = typename std::conditional<PIX == 1, uint8_t, typename std::conditional<PIX == 2, uint16_t, float>::type>::type;
-  const int xl = t;
-  if (xl >= RW) return;  // lanes past the tile's columns
   const float rounder = PIX == 4 ? 0.0f : 0.5f;
   const float fbase = (float)J.obase, norm = J.norm;
-  const int ow = J.ow, oh = J.oh, mirw = J.mirw, mirh = J.mirh, Wc = J.Wc, Hc = J.Hc, maxval = J.maxval;
-  const int interlaced = J.interlaced, half = J.Hc >> 1;
-  const long long dpitch = J.dst_pitch;
-  const int cy0 = by * stepy, cx0 = bx0 * stepx;
+  const int ow = J.ow, oh = J.oh, maxval = J.maxval;
   const int P = (int)J.seam_plane;
-  T* dpl = reinterpret_cast<T*>(dst + (long long)J.tc * dpitch + (long long)J.lc * sizeof(T));
-  const int pitch_el = (int)(dpitch / (long long)sizeof(T));
-  const int x = cx0 + xl - mirw;
-  const bool xin = x >= 0 && x < Wc;
+  T* dpl = reinterpret_cast<T*>(dst + (long long)J.tc * J.dst_pitch + (long long)J.lc * sizeof(T));
+  const float inv = 1.0f / (float)stepx;
   // x class: 0 exclusive column, 1 band inside the tile, 2 band shared with
   // the left tile (this tile holds its right block), 3 band shared with the
-  // right tile (this tile holds its left block)
-  int cls = 0, la = 0, lb = 0;
-  float wa = 0.0f, wb = 1.0f;
-  if (xl < nblk * stepx) {
-    const int bl = xl / stepx, j = xl - bl * stepx;
-    lb = bl * LSYN + j;
-    la = lb;
-    if (j < ow) {
-      wb = wsyn[XL + j];
-      if (bl >= 1) {
-        cls = 1;
-        la = (bl - 1) * LSYN + j + stepx;
-        wa = wsyn[XR + j];
-      } else {
-        cls = 2;
-      }
-    }
-  } else {
-    const int jj = xl - nblk * stepx;
-    cls = 3;
-    la = (nblk - 1) * LSYN + stepx + jj;
-    lb = la;
-    wa = wsyn[XR + jj];
-    wb = 0.0f;
+  // right tile (this tile holds its left block), 4 outside the plane
+  int cls[NQ], la[NQ], lb[NQ], x[NQ];
+  float wa[NQ], wb[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; q++) {
+    const int xq = xl + 64 * q, xt = min(xq, RW - 1);
+    x[q] = bx0 * stepx + xq - J.mirw;
+    const int bl = min(div_small(xt, stepx, inv), nblk - 1), j = xt - bl * stepx;
+    const bool right = j >= stepx;            // past the last block's body
+    const bool left = !right && j < ow;
+    const bool inner = left && bl >= 1;
+    lb[q] = bl * LSYN + j;
+    la[q] = inner ? lb[q] - LSYN + stepx : lb[q];
+    wa[q] = right ? wsyn[XR + min(j - stepx, BW - 1)] : inner ? wsyn[XR + j] : 0.0f;
+    wb[q] = right ? 0.0f : left ? wsyn[XL + j] : 1.0f;
+    cls[q] = right ? 3 : left ? (inner ? 1 : 2) : 0;
+    if (xq >= RW || x[q] < 0 || x[q] >= J.Wc) cls[q] = 4;
   }
-  const bool own = xin && cls <= 1, shr = xin && cls >= 2;
-  const int slot_x = (cls == 3 ? 0 : 1) * P;
-  const int xc = xin ? x : 0;
-#pragma unroll 8
-  for (int i = 0; i < BH; i++) {
-    const int ry = cy0 + i - mirh;
-    if (ry < 0 || ry >= Hc) continue;  // padding row (uniform)
-    const float h = syn[la + i * SYNW] * wa + syn[lb + i * SYNW] * wb;
-    const int yo = !interlaced ? ry : (ry < half ? 2 * ry : Hc - 1 - 2 * (ry - half));
-    const int so = yo * Wc + xc;
-    if (i >= oh && i < stepy) {  // rows of this block row only (uniform)
-      const float v = h * norm + rounder + fbase;
-      T q;
-      if constexpr (PIX == 4) {
-        const float o = v < 0.0f ? 0.0f : v;
-        q = o > 1.0f ? 1.0f : o;
-      } else {
-        int qi = (int)v;
-        qi = qi < 0 ? 0 : qi;
-        q = (T)(qi > maxval ? maxval : qi);
-      }
-      if (own) dpl[(unsigned)(yo * pitch_el + xc)] = q;
-      if (shr) seam[(unsigned)(slot_x + so)] = h;  // slot 0 = left block's part, slot 1 = right's
-    } else {
-      const bool ytop = i < oh;
-      const float w = wsyn[ytop ? YL + i : YR + i - stepy];
-      const int slot = cls <= 1 ? (ytop ? 1 : 0) : (ytop ? (cls == 3 ? 2 : 3) : (cls == 3 ? 0 : 1));
-      const float val = cls <= 1 ? h * (w * norm) : h;
-      if (xin) seam[(unsigned)(slot * P + so)] = val;
+  // the tile rows inside the plane
+  const int y0 = max(r0, J.mirh - by * stepy), y1 = min(r1, J.Hc + J.mirh - by * stepy);
+  auto rows = [&](int a, int b, auto&& body) {
+#pragma unroll 1
+    for (int i = a; i < b; i += RC) {
+      int ii[RC];
+      float h[NQ][RC];
+#pragma unroll
+      for (int u = 0; u < RC; u++) ii[u] = min(i + u, b - 1);
+#pragma unroll
+      for (int q = 0; q < NQ; q++)
+#pragma unroll
+        for (int u = 0; u < RC; u++) h[q][u] = syn[la[q] + ii[u] * SYNW] * wa[q] + syn[lb[q] + ii[u] * SYNW] * wb[q];
+      body(ii, h);
     }
+  };
+  // rows of two block rows: the seam buffer gets this one's part.  Row seam:
+  // slot 0 = upper block row's part, slot 1 = lower's (times its window).
+  // Corner: A upper-left, B upper-right, C lower-left, D lower-right.
+  auto band = [&](int a, int b, int yw, bool top) {
+    rows(a, b, [&](const int (&ii)[RC], const float (&h)[NQ][RC]) {
+      int o[RC];
+      float w[RC];
+#pragma unroll
+      for (int u = 0; u < RC; u++) {
+        o[u] = rowdst[ii[u]].x;
+        w[u] = wsyn[yw + ii[u]];
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        if (cls[q] == 4) continue;
+        const int slot = top ? (cls[q] <= 1 ? 1 : cls[q] == 3 ? 2 : 3) : (cls[q] == 2 ? 1 : 0);
+        const int so = slot * P + x[q];
+#pragma unroll
+        for (int u = 0; u < RC; u++) seam[(unsigned)(o[u] + so)] = cls[q] <= 1 ? h[q][u] * w[u] : h[q][u];
+      }
+    });
+  };
+  band(y0, min(y1, oh), YL, true);
+  // rows of this block row only: pixels, or, in the columns shared with the
+  // neighbouring tiles, parts (slot 0 = left block's, slot 1 = right's)
+  rows(max(y0, oh), min(y1, stepy), [&](const int (&ii)[RC], const float (&h)[NQ][RC]) {
+    int2 o[RC];
+#pragma unroll
+    for (int u = 0; u < RC; u++) o[u] = rowdst[ii[u]];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      if (cls[q] <= 1) {
+#pragma unroll
+        for (int u = 0; u < RC; u++) {
+          const float v = h[q][u] * norm + rounder + fbase;
+          T px;
+          if constexpr (PIX == 4) {
+            const float p = v < 0.0f ? 0.0f : v;
+            px = p > 1.0f ? 1.0f : p;
+          } else {
+            int qi = (int)v;
+            qi = qi < 0 ? 0 : qi;
+            px = (T)(qi > maxval ? maxval : qi);
+          }
+          dpl[(unsigned)(o[u].y + x[q])] = px;
+        }
+      } else if (cls[q] <= 3) {
+        const int so = (cls[q] == 3 ? 0 : P) + x[q];
+#pragma unroll
+        for (int u = 0; u < RC; u++) seam[(unsigned)(o[u].x + so)] = h[q][u];
+      }
+    }
+  });
+  band(max(y0, stepy), y1, YR - stepy, false);
+}
+
+// Overlap-add of the tile.  From 32 rows on, the four wavefronts take a
+// quarter of the rows each, every lane the columns 64 apart (a tile is some
+// 170 columns wide: one lane per column for all rows leaves the last
+// wavefront without work); with fewer rows, setting up several columns a lane
+// costs more than it spreads.  In thousands of cycles a 48x48 frame: 25 (one
+// lane a column, conditions and LDS reads row by row), 17 (row loops), 12 (all
+// columns together); UHD bt=5 64/16, 10 frames: 3280 -> 3000 us.
+template <int PIX, int BW, int BH, int BPW, int LSYN, int SYNW>
+__device__ __forceinline__ void overlap_cols(const PlaneJob& J, uint8_t* dst, float* seam, const float* syn,
+                                             const float* wsyn, const int2* rowdst, int by, int bx0, int nblk, int RW,
+                                             int stepx, int stepy, int t) {
+  if constexpr (BH >= 32) {
+    const int r0 = wave_of(t) * (BH / 4);
+    constexpr int NQ = (BPW * BW + 63) / 64;  // without overlap; one less is the usual case
+    if (RW <= (NQ - 1) * 64)
+      overlap_rows<PIX, BW, BH, LSYN, SYNW, NQ - 1>(J, dst, seam, syn, wsyn, rowdst, by, bx0, nblk, RW, stepx, stepy,
+                                                    t & 63, r0, r0 + BH / 4);
+    else
+      overlap_rows<PIX, BW, BH, LSYN, SYNW, NQ>(J, dst, seam, syn, wsyn, rowdst, by, bx0, nblk, RW, stepx, stepy,
+                                                t & 63, r0, r0 + BH / 4);
+  } else {
+    overlap_rows<PIX, BW, BH, LSYN, SYNW, 1>(J, dst, seam, syn, wsyn, rowdst, by, bx0, nblk, RW, stepx, stepy, t, 0,
+                                             BH);
   }
 }
 
@@ -386,6 +468,8 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
   __shared__ __align__(16) float wsyn[2 * BW + 2 * BH];  // synthesis windows: left, right, top, bottom bands
   // byte offset of the source row of each tile row (< 2^31: checked by the host)
   __shared__ __align__(16) int rowoff[BH];
+  // element offsets of each tile row in a seam plane and in the destination
+  __shared__ __align__(16) int2 rowdst[BH];
   float2* spec = reinterpret_cast<float2*>(smem);
   float2* stage = reinterpret_cast<float2*>(smem);
   float* syn = reinterpret_cast<float*>(smem);
@@ -409,18 +493,28 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
       // (the FFT form's row transforms take halved samples: exact)
       winy[i] = MF ? J.wany[i] : 0.5f * J.wany[i];
       rowoff[i] = (int)((long long)(cover_to_src_row(J, by * stepy + i) + J.tc) * J.src_pitch);
+      const int yo = interior_to_out_row(J, by * stepy + i - J.mirh);  // (used inside the plane only)
+      rowdst[i] = make_int2(yo * J.Wc, yo * (int)(J.dst_pitch / (long long)J.pix));
     }
     for (int i = t; i < J.ow; i += NT) {
       wsyn[i] = J.wsynxl[i];
       wsyn[BW + i] = J.wsynxr[i];
     }
     for (int i = t; i < J.oh; i += NT) {
-      wsyn[2 * BW + i] = J.wsynyl[i];
-      wsyn[2 * BW + BH + i] = J.wsynyr[i];
+      wsyn[2 * BW + i] = J.wsynyl[i] * J.norm;
+      wsyn[2 * BW + BH + i] = J.wsynyr[i] * J.norm;
     }
   }
   __syncthreads();
 
+  // Wiener 3D loads a frame's samples ahead, to be in flight during the
+  // overlap-add of the frame before (48x48: 7.9 of 69 thousand cycles of a
+  // frame were that wait; 1080p 64 frames 2416 -> 2372 us).  The other modes
+  // have the registers for more wavefronts instead, which hide it as well
+  // (Kalman), or one frame a workgroup (2D).
+  constexpr bool AHEAD = MODE == MODE_W3D;
+  uint32_t raw[BH];
+  if constexpr (AHEAD) gather_load<BW, BH>(L0.J, raw, L0.src[i0], rowoff, bx0, nblk, stepx, (int)threadIdx.x);
 #pragma unroll 1
   for (int fi = i0; fi < i1; fi++) {
     // The lane index, the launch record and the LDS tables are reached
@@ -437,7 +531,6 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     const float* wy = winy + zo;
     const int* ro = rowoff + zo;
     const int m = L.m0 + fi;
-    const int pix = J.pix;
     // column lanes: a pair (l, l + 32) per column, half hh: rows hh * CR/2 + i
     // and BH/2 + hh * CR/2 + i, i < CR/2, of the spectrum after the forward
     // transform (value j of the lane: row hh * CR/2 + col_row(j))
@@ -462,16 +555,9 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     const SpecParams SP(J);
 
     // ---- 1. windowed pixels into per-block row pairs
-    const uint8_t* fsrc = L.src[fi];
-    if (MF && (by == 0 || by == J.noy - 1)) {
-      if (pix == 1) gather_cols<1, BW, BH, SA, LA, MF>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
-      else if (pix == 2) gather_cols<2, BW, BH, SA, LA, MF>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
-      else gather_cols<4, BW, BH, SA, LA, MF>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
-    } else {
-      if (pix == 1) gather_cols<1, BW, BH, SA, LA, false>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
-      else if (pix == 2) gather_cols<2, BW, BH, SA, LA, false>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
-      else gather_cols<4, BW, BH, SA, LA, false>(J, stage, fsrc, ro, wx, wy, by, bx0, nblk, stepx, t);
-    }
+    if constexpr (!AHEAD) gather_load<BW, BH>(J, raw, L.src[fi], ro, bx0, nblk, stepx, t);
+    if (MF && (by == 0 || by == J.noy - 1)) gather_window<BW, BH, SA, LA, MF>(J, stage, raw, wx, wy, by, bx0, nblk, t);
+    else gather_window<BW, BH, SA, LA, false>(J, stage, raw, wx, wy, by, bx0, nblk, t);
     __syncthreads();
     if constexpr (MF) {
       // ---- 2-3. 2D r2c on the matrix cores, in rounds of one block per
@@ -776,26 +862,21 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
       }
     }
     __syncthreads();
+    if constexpr (AHEAD) {
+      // (after the last frame nothing: an undefined value would stay alive)
+      if (fi + 1 < i1) gather_load<BW, BH>(J, raw, L.src[fi + 1], ro, bx0, nblk, stepx, t);
+      else static_for<0, BH>([&](auto i) { raw[i] = 0; });
+    }
     // ---- 7. overlap-add inside the tile; seam partials to this frame's seam buffer
     uint8_t* dst = L.dst[fi];
     float* seam = J.seam + (size_t)fi * 4 * (size_t)J.seam_plane;
     const float* ws = wsyn + zo;
-    if (pix == 1) overlap_cols<1, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-    else if (pix == 2) overlap_cols<2, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
-    else overlap_cols<4, BW, BH, LSYN, SYNW>(J, dst, seam, syn, ws, by, bx0, nblk, RW, stepx, stepy, t);
+    const int2* rd = rowdst + zo;
+    if (J.pix == 1) overlap_cols<1, BW, BH, BPW, LSYN, SYNW>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
+    else if (J.pix == 2) overlap_cols<2, BW, BH, BPW, LSYN, SYNW>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
+    else overlap_cols<4, BW, BH, BPW, LSYN, SYNW>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
     __syncthreads();  // syn read; the next frame's gather writes the stage
   }
-}
-
-// n / d for 0 <= n < 2^22 and 1 <= d <= 64 (inv = 1/d rounded): the float
-// quotient is within one of the exact one, and one correction each way
-// makes it exact.
-__device__ __forceinline__ int div_small(int n, int d, float inv) {
-  int q = (int)((float)n * inv);
-  const int r = n - q * d;
-  q += r >= d ? 1 : 0;
-  q -= r < 0 ? 1 : 0;
-  return q;
 }
 
 // Seam pixels of every frame of a k_run launch, finished from the partial

@@ -179,11 +179,8 @@ template <int BT, class PJ>
 __device__ __forceinline__ float2 apply3d_elem(const PJ& J, const float2 (&v)[5], const Tab& T, float gf) {
   const float sig = T.sig;
   const float ll = J.lowlimit;
-  float g0 = 0.0f, g1 = 0.0f;
-  if (J.use_degrid) {
-    g0 = gf * T.g.x * (float)BT;
-    g1 = gf * T.g.y * (float)BT;
-  }
+  // without degrid the fraction gf is zero, and so are these
+  const float g0 = gf * T.g.x * (float)BT, g1 = gf * T.g.y * (float)BT;
   // the temporal DFT of the reference's formulas, the Wiener gain of each
   // bin, and the inverse at the current frame as one fused sum per part
   float2 r;
