@@ -210,10 +210,16 @@ struct nf3d_engine {
   int out_stride = 0;
   std::mutex mu;
   // Ordering between calls on different streams: the work of the last call
-  // ends with done_ev on done_stream, and a call on another stream waits for
+  // ends with the event of `done` on done_stream, and a call on another stream waits for
   // it first (the spectra ring, the Kalman state and the seam and staging
   // buffers carry over from one call to the next).
-  hipEvent_t done_ev = nullptr;
+  struct Mark {
+    hipEvent_t ev = nullptr;
+    ~Mark() {
+      if (ev) (void)hipEventDestroy(ev);
+    }
+  };
+  std::shared_ptr<Mark> own_mark, done;  // (done: this engine's or its batch's first engine's)
   hipStream_t done_stream = nullptr;
   // opt-in HIP-event timing of the main spectral kernel of each frame
   bool profiling = false;
@@ -295,7 +301,6 @@ struct nf3d_engine {
     for (auto* p : h_up) hipHostFree(p);
     hipHostFree(h_down);
     for (auto ev : ev_pool) hipEventDestroy(ev);
-    if (done_ev) hipEventDestroy(done_ev);
     if (stream) hipStreamDestroy(stream);
   }
 
@@ -702,12 +707,25 @@ struct nf3d_engine {
   // A call on stream s starts after the previous call's work (if that went
   // to another stream) ...
   void order_before(hipStream_t s) {
-    if (done_stream && done_stream != s) check(hipStreamWaitEvent(s, done_ev, 0), "hipStreamWaitEvent");
+    if (done_stream && done_stream != s) check(hipStreamWaitEvent(s, done->ev, 0), "hipStreamWaitEvent");
   }
-  // ... and marks its own end.
+  // ... and marks its own end: one event for all engines of a batch (an event
+  // each cost 4 us of the stream's time).  The event is the first engine's,
+  // shared with the others; when that engine records it again for a later call
+  // of its own, that call has come after the batch's work, so a wait for the
+  // event still covers it.
   void order_after(hipStream_t s) {
-    if (!done_ev) check(hipEventCreateWithFlags(&done_ev, hipEventDisableTiming), "hipEventCreate");
-    check(hipEventRecord(done_ev, s), "hipEventRecord");
+    if (!own_mark) {
+      auto m = std::make_shared<Mark>();
+      check(hipEventCreateWithFlags(&m->ev, hipEventDisableTiming), "hipEventCreate");
+      own_mark = m;
+    }
+    check(hipEventRecord(own_mark->ev, s), "hipEventRecord");
+    done = own_mark;
+    done_stream = s;
+  }
+  void order_after(hipStream_t s, const nf3d_engine& first) {
+    done = first.done;
     done_stream = s;
   }
 
@@ -1065,10 +1083,15 @@ struct nf3d_engine {
     // learned PSD: launch j predicts (else it keeps its span's PSD in d_lpat)
     std::vector<char> predict;
     // Wiener 3D: the clip-end frames of the range (btcur 1, the 2D gains)
-    // as one-frame launches of the frame-loop kernel in its 2D mode, instead
-    // of the per-frame path: those before the frame-loop frames (run after
-    // the prologue, while the ring still holds them) and those after
+    // as launches of the frame-loop kernel in its 2D mode, a frame per
+    // workgroup, instead of the per-frame path: those before the frame-loop
+    // frames (run after the prologue, while the ring still holds them) and
+    // those after, each in one launch (a learned PSD is predicted per launch,
+    // from its frame: one frame each)
     std::vector<RunLaunch> edges_start, edges;
+    // Wiener 3D: the forward transforms of the first window's older frames
+    // that the ring does not hold (none, or one launch)
+    std::vector<RunLaunch> fwd;
   };
 
   RangePlan plan_range(int first, int count, const void* const* src, long long src_pitch, void* const* dst,
@@ -1164,26 +1187,31 @@ struct nf3d_engine {
     if (P.mode == nf3d::MODE_W3D) {
       for (int n = first; n < first + count; n++) {
         if (n >= P.a && n <= P.b) continue;
-        RunLaunch R = run_job();
-        R.J.sigma2 = ep.sigma * ep.sigma / norm;  // btcur = 1 (src/fft3d_engine.h's window rule)
-        R.J.seam = d_seam_run;  // the edge launches run apart from the others on the stream
-        if (learned) use_learned(R.J);
-        R.J.src_pitch = src_pitch;
-        R.J.dst_pitch = dst_pitch;
-        R.src[0] = static_cast<const uint8_t*>(src[n]);
-        R.dst[0] = static_cast<uint8_t*>(dst[n]);
-        R.m0 = n;
-        R.nframes = 1;
-        R.fpw = 1;
-        (n < P.a ? P.edges_start : P.edges).push_back(R);
+        std::vector<RunLaunch>& E = n < P.a ? P.edges_start : P.edges;
+        if (E.empty() || learned || E.back().nframes == kRunFrames) {
+          RunLaunch R = run_job();
+          R.J.sigma2 = ep.sigma * ep.sigma / norm;  // btcur = 1 (src/fft3d_engine.h's window rule)
+          R.J.seam = d_seam_run;  // the edge launches run apart from the others on the stream
+          if (learned) use_learned(R.J);
+          R.J.src_pitch = src_pitch;
+          R.J.dst_pitch = dst_pitch;
+          R.m0 = n;
+          R.fpw = 1;
+          E.push_back(R);
+        }
+        RunLaunch& R = E.back();
+        R.src[R.nframes] = static_cast<const uint8_t*>(src[n]);
+        R.dst[R.nframes] = static_cast<uint8_t*>(dst[n]);
+        R.nframes++;
       }
     }
     return P;
   }
 
   // Frames before the frame-loop launches (or all, without them), the
-  // pattern estimate, the Wiener-3D ring slots of the first window.
-  void run_prologue(const RangePlan& P, hipStream_t s) {
+  // pattern estimate, and the plan of the Wiener-3D ring slots of the first
+  // window (P.fwd, launched for all engines of a batch together).
+  void run_prologue(RangePlan& P, hipStream_t s) {
     check(hipSetDevice(device), "hipSetDevice");
     const int stop = P.run ? P.a : P.first + P.count;
     if (P.edges.empty() && P.edges_start.empty())
@@ -1203,9 +1231,7 @@ struct nf3d_engine {
       int k0 = P.a + P.from;
       while (k0 < P.a + P.to && ring_frame[k0 % ep.bt] == k0 && ring_by_run[k0 % ep.bt]) k0++;
       if (k0 < P.a + P.to) {
-        nf3d::RunBatch B{};
-        RunLaunch& R = B.job[0];
-        R = run_job();
+        RunLaunch R = run_job();
         R.J.src_pitch = P.src_pitch;
         R.J.dst_pitch = P.dst_pitch;
         for (int k = k0; k < P.a + P.to; k++) R.src[k - k0] = static_cast<const uint8_t*>(P.src[k]);
@@ -1213,21 +1239,20 @@ struct nf3d_engine {
         R.spec_elems = (long long)spec_elems;
         R.m0 = k0;
         R.nframes = P.a + P.to - k0;
-        R.fpw = R.nframes;
-        R.wg_begin = 0;
-        B.njobs = 1;
-        B.total_wg = R.ntiles;
-        B.max_hc = Hc;
-        B.max_frames = R.nframes;
-        check(nf3d::launch_run(nf3d::MODE_FWD, ep.bt, nf3d::SHP_NONE, dft_mode, ep.bw, ep.bh, B, s),
-              "frame-loop forward transforms");
-        for (int k = k0; k < P.a + P.to; k++) {
-          ring_frame[k % ep.bt] = k;
-          ring_by_run[k % ep.bt] = 1;
-          ring_tick[k % ep.bt] = ++tick;
-        }
+        R.fpw = 1;  // (the frames are independent)
+        P.fwd.push_back(R);
       }
     }
+  }
+
+  // Ring bookkeeping after the launch of P.fwd.
+  void fwd_launched(const RangePlan& P) {
+    for (const RunLaunch& R : P.fwd)
+      for (int k = R.m0; k < R.m0 + R.nframes; k++) {
+        ring_frame[k % ep.bt] = k;
+        ring_by_run[k % ep.bt] = 1;
+        ring_tick[k % ep.bt] = ++tick;
+      }
   }
 
   // Ring bookkeeping after the frame-loop launches, then the frames after them.
@@ -1517,11 +1542,13 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
     const nf3d_run_item& it = items[i];
     plans[i] = it.engine->plan_range(it.first, it.count, it.src, it.src_stride, it.dst, it.dst_stride);
   }
-  // the clip-end frames of Wiener-3D ranges: one-frame launches of the
-  // frame-loop kernel in its 2D mode, engines of the same shape, sharpen
-  // case and transform form together (those before the frame-loop frames
-  // right after the prologues, the others after the frame-loop launches)
-  auto run_edges = [&](std::vector<RunLaunch> nf3d_engine::RangePlan::*which) {
+  // the launches before and after the frame-loop ones, engines of the same
+  // shape, sharpen case and transform form (forward transforms: and bt)
+  // together: the forward transforms of the first windows, and the clip-end
+  // frames in the 2D mode (those before the frame-loop frames right after the
+  // prologues, the others after the frame-loop launches)
+  auto run_apart = [&](std::vector<RunLaunch> nf3d_engine::RangePlan::*which, int mode) {
+    const bool fwd = mode == nf3d::MODE_FWD;
     std::vector<bool> edone(n, false);
     for (int i = 0; i < n; i++) {
       if (edone[i] || (plans[i].*which).empty()) continue;
@@ -1530,7 +1557,7 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
       for (int k = i; k < n; k++) {
         nf3d_engine* e = items[k].engine;
         if (!edone[k] && !(plans[k].*which).empty() && e->ep.bw == e0->ep.bw && e->ep.bh == e0->ep.bh &&
-            plans[k].shp == plans[i].shp && e->dft_mode == e0->dft_mode) {
+            (fwd ? e->ep.bt == e0->ep.bt : plans[k].shp == plans[i].shp) && e->dft_mode == e0->dft_mode) {
           group.push_back(k);
           edone[k] = true;
         }
@@ -1550,13 +1577,19 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
             RunLaunch& R = B.job[B.njobs++];
             R = (plans[k].*which)[q];
             R.wg_begin = B.total_wg;
-            B.total_wg += R.ntiles;
+            B.total_wg += R.ntiles * R.nframes;
             B.max_hc = std::max(B.max_hc, e->Hc);
-            B.max_frames = 1;
+            B.max_frames = std::max(B.max_frames, R.nframes);
           }
-          learned_predictions(items, plans, members, c0, B, nf3d::MODE_W2D, SIZE_MAX, s);
-          for (int c = 0; c < B.njobs; c++) evs.push_back(items[members[c0 + c]].engine->timer(timed, 1, s));
-          check(nf3d::launch_run(nf3d::MODE_W2D, 0, plans[i].shp, e0->dft_mode, e0->ep.bw, e0->ep.bh, B, s),
+          if (fwd) {
+            check(nf3d::launch_run(mode, e0->ep.bt, nf3d::SHP_NONE, e0->dft_mode, e0->ep.bw, e0->ep.bh, B, s),
+                  "frame-loop forward transforms");
+            continue;
+          }
+          learned_predictions(items, plans, members, c0, B, mode, SIZE_MAX, s);
+          for (int c = 0; c < B.njobs; c++)
+            evs.push_back(items[members[c0 + c]].engine->timer(timed, B.job[c].nframes, s));
+          check(nf3d::launch_run(mode, 0, plans[i].shp, e0->dft_mode, e0->ep.bw, e0->ep.bh, B, s),
                 "frame-loop kernel (clip ends)");
           check(nf3d::launch_seam_run(e0->dft_mode, e0->ep.bw, e0->ep.bh, B, s), "seam kernel");
           for (auto& ev : evs)
@@ -1566,7 +1599,9 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
     }
   };
   for (int i = 0; i < n; i++) items[i].engine->run_prologue(plans[i], s);
-  run_edges(&nf3d_engine::RangePlan::edges_start);
+  run_apart(&nf3d_engine::RangePlan::fwd, nf3d::MODE_FWD);
+  for (int i = 0; i < n; i++) items[i].engine->fwd_launched(plans[i]);
+  run_apart(&nf3d_engine::RangePlan::edges_start, nf3d::MODE_W2D);
   // the frame-loop launches, grouped by block shape, mode, bt, sharpen case
   // and transform form
   std::vector<std::vector<int>> groups;
@@ -1652,11 +1687,13 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
       check(hipStreamWaitEvent(s, j, 0), "hipStreamWaitEvent");
     }
   }
-  run_edges(&nf3d_engine::RangePlan::edges);
+  run_apart(&nf3d_engine::RangePlan::edges, nf3d::MODE_W2D);
   for (int i = 0; i < n; i++) items[i].engine->run_epilogue(plans[i], s);
   for (int i = 0; i < n; i++) items[i].engine->last_end = items[i].first + items[i].count - 1;
   if (!capture)
-    for (int i = 0; i < n; i++) items[i].engine->order_after(s);
+    for (int i = 0; i < n; i++)
+      if (i == 0) items[0].engine->order_after(s);
+      else items[i].engine->order_after(s, *items[0].engine);
 }
 
 // Locks every engine of a batch (address order), after checking the items.
@@ -2206,7 +2243,9 @@ int nf3d_graph_launch(nf3d_graph* g, void* stream) {
   try {
     for (nf3d_engine* e : g->engines) e->order_before(s);
     check(hipGraphLaunch(g->exec, s), "hipGraphLaunch");
-    for (nf3d_engine* e : g->engines) e->order_after(s);
+    for (nf3d_engine* e : g->engines)
+      if (e == g->engines[0]) e->order_after(s);
+      else e->order_after(s, *g->engines[0]);
   } catch (const Failure&) {
     return -1;
   }
@@ -2475,7 +2514,7 @@ int nf3d_engine_profile_read(nf3d_engine* e, double* total_ms, int* frames) {
 int nf3d_engine_sync(nf3d_engine* e) {
   std::lock_guard<std::mutex> lock(e->mu);
   if (hipStreamSynchronize(e->stream) != hipSuccess) return -1;
-  if (e->done_ev && hipEventSynchronize(e->done_ev) != hipSuccess) return -1;
+  if (e->done && hipEventSynchronize(e->done->ev) != hipSuccess) return -1;
   return 0;
 }
 
