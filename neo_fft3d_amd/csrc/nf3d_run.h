@@ -266,14 +266,19 @@ __device__ __forceinline__ void overlap_rows(const PlaneJob& J, uint8_t* dst, fl
 // costs more than it spreads.  In thousands of cycles a 48x48 frame: 25 (one
 // lane a column, conditions and LDS reads row by row), 17 (row loops), 12 (all
 // columns together); UHD bt=5 64/16, 10 frames: 3280 -> 3000 us.
-template <int PIX, int BW, int BH, int BPW, int LSYN, int SYNW>
+template <int PIX, int BW, int BH, int BPW, int LSYN, int SYNW, int QM>
 __device__ __forceinline__ void overlap_cols(const PlaneJob& J, uint8_t* dst, float* seam, const float* syn,
                                              const float* wsyn, const int2* rowdst, int by, int bx0, int nblk, int RW,
                                              int stepx, int stepy, int t) {
   if constexpr (BH >= 32) {
     const int r0 = wave_of(t) * (BH / 4);
     constexpr int NQ = (BPW * BW + 63) / 64;  // without overlap; one less is the usual case
-    if (RW <= (NQ - 1) * 64)
+    if constexpr (QM < NQ) {  // (fewer registers)
+#pragma unroll 1
+      for (int x0 = 0; x0 < RW; x0 += 64 * QM)
+        overlap_rows<PIX, BW, BH, LSYN, SYNW, QM>(J, dst, seam, syn, wsyn, rowdst, by, bx0, nblk, RW, stepx, stepy,
+                                                  x0 + (t & 63), r0, r0 + BH / 4);
+    } else if (RW <= (NQ - 1) * 64)
       overlap_rows<PIX, BW, BH, LSYN, SYNW, NQ - 1>(J, dst, seam, syn, wsyn, rowdst, by, bx0, nblk, RW, stepx, stepy,
                                                     t & 63, r0, r0 + BH / 4);
     else
@@ -429,16 +434,23 @@ __device__ __forceinline__ void split_combine_inv(float2 (&c)[N / 2], int h) {
 // per CU at 48x48): three, or two for the variants whose spectral pass holds
 // more per element (four or five frames, the dehalo factor, the Kalman state
 // with a sharpen pass, 64-row columns), which would otherwise spill.
-template <int BH, int MODE, int BT, int SHP>
+template <int BH, int MODE, int BT, int SHP, bool RES>
 constexpr int run_waves_per_simd() {
   if constexpr (BH >= 64 || (MODE == MODE_W3D && (BT >= 4 || SHP == SHP_GENERAL)) ||
-                (MODE == MODE_KALMAN && SHP != SHP_NONE))
+                (MODE == MODE_KALMAN && (SHP != SHP_NONE || (RES && BH > 32))))
     return 2;
   else return 3;
 }
 
-template <int BW, int BH, int NT, int MODE, int BT, int SHP, bool MF = false>
-__global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>())) k_run(RunBatch B_arg) {
+//
+// RES (Kalman): a lane keeps its elements' state in registers from the first
+// frame of a launch to its last (12 bytes an element: 48 registers at 32x32,
+// 72 at 48x48) instead of reading and writing it for every frame: UHD 4:2:0
+// 10-bit, 11 frames a launch, 8x8 1289 -> 814 us, 16x16 1569 -> 953, 24x24
+// 1530 -> 1092, 32x32 1452 -> 1141, 48x48 1477 -> 1347.  At 64x64 96 more do
+// not fit (344 bytes of scratch a lane: 1649 -> 2437).
+template <int BW, int BH, int NT, int MODE, int BT, int SHP, bool MF = false, bool RES = false>
+__global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP, RES>())) k_run(RunBatch B_arg) {
   const RunBatch& B0 = kernarg_batch(B_arg);
   const int jb = batch_job(B0, blockIdx.x);
   const RunLaunch& L0 = B0.job[jb];
@@ -515,6 +527,19 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
   constexpr bool AHEAD = MODE == MODE_W3D;
   uint32_t raw[BH];
   if constexpr (AHEAD) gather_load<BW, BH>(L0.J, raw, L0.src[i0], rowoff, bx0, nblk, stepx, (int)threadIdx.x);
+  // the lane's Kalman state (RES; lanes past the tile's columns hold a copy of
+  // one of them, and store nothing)
+  static_assert(!RES || MODE == MODE_KALMAN, "the resident state is the Kalman mode's");
+  KalState kst[RES ? CR : 1];
+  auto state_at = [&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    const int t = threadIdx.x, cl = (t >> 6) * 32 + (t & 31), hh = (t >> 5) & 1;
+    const int cbr = cl / COLS, cc = cl - cbr * COLS, cb = min(cbr, nblk - 1);
+    return ((size_t)(by * L0.J.nox + bx0) + cb) * (BH * COLS) +
+           (size_t)(hh * (CR / 2) + i + (i >= CR / 2 ? CR / 2 : 0)) * COLS + cc;
+  };
+  if constexpr (RES)
+    static_for<0, CR>([&](auto i) { kst[i] = KalState{L0.J.kal_last[state_at(i)], L0.J.kal_sum[state_at(i)]}; });
 #pragma unroll 1
   for (int fi = i0; fi < i1; fi++) {
     // The lane index, the launch record and the LDS tables are reached
@@ -663,7 +688,7 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
         constexpr int u = decltype(uu)::value, i = k * CH + u;
         const size_t o = colo + (size_t)col_row(std::integral_constant<int, i>{}) * COLS;
         static_for<0, NQ>([&](auto qq) { b.v[decltype(qq)::value][u] = rq[decltype(qq)::value][o]; });
-        if constexpr (MODE == MODE_KALMAN) b.ks[u] = KalState{J.kal_last[o], J.kal_sum[o]};
+        if constexpr (MODE == MODE_KALMAN && !RES) b.ks[u] = KalState{J.kal_last[o], J.kal_sum[o]};
       });
     };
     const int tab0 = hh * (CR / 2) * COLS + cc;  // table element of the lane's first row
@@ -729,7 +754,9 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
         gf = J.use_degrid ? J.degrid * col[0].x / grid0 : 0.0f;
         dcf = apply2d_s<SHP>(SP, col[0], T0, gf).x;
       } else if constexpr (MODE == MODE_KALMAN) {
-        KalState st = rbuf[0].ks[0];
+        KalState st;
+        if constexpr (RES) st = kst[0];
+        else st = rbuf[0].ks[0];
         dcf = kalman_elem(SP, col[0], T0, st).x;
       } else {
         dcf = col[0].x;
@@ -766,9 +793,13 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
               r = SP.use_pattern ? rs : r;
             }
           } else if constexpr (MODE == MODE_KALMAN) {
-            KalState st = b.ks[u];
+            KalState st;
+            if constexpr (RES) st = kst[i];
+            else st = b.ks[u];
             r = kalman_elem(SP, col[i], T, st);
-            if (col_on) {
+            if constexpr (RES) {
+              kst[i] = st;
+            } else if (col_on) {
               const size_t o = colo + (size_t)col_row(std::integral_constant<int, i>{}) * COLS;
               J.kal_last[o] = st.last;
               J.kal_sum[o] = st.sum;
@@ -872,10 +903,18 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP>()))
     float* seam = J.seam + (size_t)fi * 4 * (size_t)J.seam_plane;
     const float* ws = wsyn + zo;
     const int2* rd = rowdst + zo;
-    if (J.pix == 1) overlap_cols<1, BW, BH, BPW, LSYN, SYNW>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
-    else if (J.pix == 2) overlap_cols<2, BW, BH, BPW, LSYN, SYNW>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
-    else overlap_cols<4, BW, BH, BPW, LSYN, SYNW>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
+    if (J.pix == 1) overlap_cols<1, BW, BH, BPW, LSYN, SYNW, RES ? 2 : 4>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
+    else if (J.pix == 2) overlap_cols<2, BW, BH, BPW, LSYN, SYNW, RES ? 2 : 4>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
+    else overlap_cols<4, BW, BH, BPW, LSYN, SYNW, RES ? 2 : 4>(J, dst, seam, syn, ws, rd, by, bx0, nblk, RW, stepx, stepy, t);
     __syncthreads();  // syn read; the next frame's gather writes the stage
+  }
+  if constexpr (RES) {
+    const int t = threadIdx.x, cl = (t >> 6) * 32 + (t & 31);
+    if (cl / COLS < nblk)
+      static_for<0, CR>([&](auto i) {
+        L0.J.kal_last[state_at(i)] = kst[i].last;
+        L0.J.kal_sum[state_at(i)] = kst[i].sum;
+      });
   }
 }
 
@@ -953,6 +992,8 @@ hipError_t launch_run_modes(int mode, int bt, int shp, const RunBatch& L, hipStr
   constexpr int NT = 256;
   dim3 grid(L.total_wg), block(NT);
 #define NF3D_RUN(M, B, H) hipLaunchKernelGGL((k_run<BW, BH, NT, M, B, H, MF>), grid, block, 0, s, L)
+#define NF3D_RUN_RES(H) \
+  hipLaunchKernelGGL((k_run<BW, BH, NT, MODE_KALMAN, 0, H, false, true>), grid, block, 0, s, L)
 #define NF3D_RUN_SHP(M, B)                                   \
   switch (shp) {                                             \
     case SHP_NONE: NF3D_RUN(M, B, SHP_NONE); break;          \
@@ -971,7 +1012,24 @@ hipError_t launch_run_modes(int mode, int bt, int shp, const RunBatch& L, hipStr
       }
       break;
     case MODE_W2D: NF3D_RUN_SHP(MODE_W2D, 0); break;
-    case MODE_KALMAN: NF3D_RUN_SHP(MODE_KALMAN, 0); break;
+    case MODE_KALMAN:
+      // the state stays in registers where a launch has the frames to make up
+      // for loading it all at once at the start (one frame: 32x32 177 -> 184
+      // us) and, at 48x48, for two instead of three wavefronts a SIMD (one
+      // frame: 193 -> 213 us)
+      if constexpr (!MF && BH <= 48) {
+        if (L.max_frames >= (BH <= 32 ? 2 : 4)) {
+          switch (shp) {
+            case SHP_NONE: NF3D_RUN_RES(SHP_NONE); break;
+            case SHP_SHARPEN: NF3D_RUN_RES(SHP_SHARPEN); break;
+            case SHP_GENERAL: NF3D_RUN_RES(SHP_GENERAL); break;
+            default: return hipErrorInvalidValue;
+          }
+          break;
+        }
+      }
+      NF3D_RUN_SHP(MODE_KALMAN, 0);
+      break;
     case MODE_SHARPEN:
       if (shp == SHP_SHARPEN) NF3D_RUN(MODE_SHARPEN, 0, SHP_SHARPEN);
       else if (shp == SHP_GENERAL) NF3D_RUN(MODE_SHARPEN, 0, SHP_GENERAL);
@@ -989,6 +1047,7 @@ hipError_t launch_run_modes(int mode, int bt, int shp, const RunBatch& L, hipStr
     default: return hipErrorInvalidValue;
   }
 #undef NF3D_RUN_SHP
+#undef NF3D_RUN_RES
 #undef NF3D_RUN
   return hipGetLastError();
 }
