@@ -78,47 +78,58 @@ __device__ __forceinline__ float gelu_grad(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-// One operand tile (R rows of the outer index x 64 k) as R*8 chunks of 8
-// contiguous elements; each lane loads R*8/256 of them.  KC: k is the
-// contiguous index in memory (row-major A, transposed B), else the outer
-// index is.
+// One operand tile (R rows of the outer index x 64 k), k contiguous in LDS.
+// KC: k is the contiguous index in memory too (row-major A, transposed B) and
+// a lane moves R*8/256 chunks of 8 elements.
 template <bool KC, int R>
 struct TileLoad {
   static constexpr int NCH = R * 8 / NT;
-  static constexpr int OC = R / 8;  // chunks per k-row when the outer index is contiguous
   uint4 v[NCH];
   __device__ void load(const __bf16* P, long long ld, int o0, int olim, int k0, int klim, int t) {
 #pragma unroll
     for (int h = 0; h < NCH; h++) {
-      const int c = t + h * NT;
-      int o, k;
-      if constexpr (KC) {
-        o = c >> 3;
-        k = (c & 7) * 8;
-      } else {
-        k = c / OC;
-        o = (c % OC) * 8;
-      }
-      const int go = o0 + o, gk = k0 + k;
+      const int c = t + h * NT, go = o0 + (c >> 3), gk = k0 + (c & 7) * 8;
       v[h] = make_uint4(0, 0, 0, 0);
-      if (go < olim && gk < klim)
-        v[h] = *reinterpret_cast<const uint4*>(KC ? P + (long long)go * ld + gk : P + (long long)gk * ld + go);
+      if (go < olim && gk < klim) v[h] = *reinterpret_cast<const uint4*>(P + (long long)go * ld + gk);
     }
   }
   __device__ void store(__bf16* S, int t) const {
 #pragma unroll
     for (int h = 0; h < NCH; h++) {
       const int c = t + h * NT;
-      if constexpr (KC) {
-        *reinterpret_cast<uint4*>(S + (c >> 3) * LDK + (c & 7) * 8) = v[h];
-      } else {
-        const int k = c / OC, o = (c % OC) * 8;
-        __bf16 e[8];
-        memcpy(e, &v[h], 16);
-#pragma unroll
-        for (int i = 0; i < 8; i++) S[(o + i) * LDK + k] = e[i];
-      }
+      *reinterpret_cast<uint4*>(S + (c >> 3) * LDK + (c & 7) * 8) = v[h];
     }
+  }
+};
+// The outer index contiguous in memory (the operands of a weight gradient,
+// whose k is the batch row): a lane takes 4 outer elements of 4 k rows and
+// turns them in registers, so LDS gets 4 stores of 8 bytes for 16 elements, a
+// wavefront's on all 64 banks alike, where element stores of 2 bytes met on
+// 16 banks and bounded the product (the three weight gradients of 4096 rows
+// through 1200-256-256-1200: 77 -> 51 us).  R = 32 has work for 128 lanes: the
+// kernel gives the two operands to different wavefronts.
+template <int R>
+struct TileLoad<false, R> {
+  static_assert(R * 4 <= NT, "one unit a lane");
+  uint2 v[4];
+  __device__ void load(const __bf16* P, long long ld, int o0, int olim, int k0, int klim, int t) {
+    if (t >= R * 4) return;
+    const int go = o0 + (t % (R / 4)) * 4, gk = k0 + (t / (R / 4)) * 4;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      v[j] = make_uint2(0, 0);
+      if (go < olim && gk + j < klim) v[j] = *reinterpret_cast<const uint2*>(P + (long long)(gk + j) * ld + go);
+    }
+  }
+  __device__ void store(__bf16* S, int t) const {
+    if (t >= R * 4) return;
+    __bf16* d = S + (t % (R / 4)) * 4 * LDK + (t / (R / 4)) * 4;
+    auto lo = [](unsigned a, unsigned b) { return (a & 0xffffu) | (b << 16); };
+    auto hi = [](unsigned a, unsigned b) { return (a >> 16) | (b & 0xffff0000u); };
+    *reinterpret_cast<uint2*>(d) = make_uint2(lo(v[0].x, v[1].x), lo(v[2].x, v[3].x));
+    *reinterpret_cast<uint2*>(d + LDK) = make_uint2(hi(v[0].x, v[1].x), hi(v[2].x, v[3].x));
+    *reinterpret_cast<uint2*>(d + 2 * LDK) = make_uint2(lo(v[0].y, v[1].y), lo(v[2].y, v[3].y));
+    *reinterpret_cast<uint2*>(d + 3 * LDK) = make_uint2(hi(v[0].y, v[1].y), hi(v[2].y, v[3].y));
   }
 };
 
@@ -127,14 +138,14 @@ __global__ void __launch_bounds__(NT) k_gemm(GemmArgs g) {
   constexpr int MI = TM / 32, NJ = TN / 32;  // 16x16 MFMA tiles per wave
   __shared__ __attribute__((aligned(16))) __bf16 As[TM * LDK];
   __shared__ __attribute__((aligned(16))) __bf16 Bs[TN * LDK];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = threadIdx.x, tb = t ^ (NT / 2), lane = t & 63, w = t >> 6;
   const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
   const int wm = (w & 1) * (TM / 2), wn = (w >> 1) * (TN / 2);
   const int kb = blockIdx.z * g.kc, ke = min(g.K, kb + g.kc);
   TileLoad<!TA, TM> la;
   TileLoad<TB, TN> lb;
   la.load(g.A, g.lda, m0, g.M, kb, ke, t);
-  lb.load(g.B, g.ldb, n0, g.N, kb, ke, t);
+  lb.load(g.B, g.ldb, n0, g.N, kb, ke, tb);
   f32x4 acc[MI][NJ];
 #pragma unroll
   for (int i = 0; i < MI; i++)
@@ -144,11 +155,11 @@ __global__ void __launch_bounds__(NT) k_gemm(GemmArgs g) {
   for (int k0 = kb; k0 < ke; k0 += TK) {
     __syncthreads();  // the previous step's MFMAs are done with the tiles
     la.store(As, t);
-    lb.store(Bs, t);
+    lb.store(Bs, tb);
     __syncthreads();
     if (k0 + TK < ke) {
       la.load(g.A, g.lda, m0, g.M, k0 + TK, ke, t);
-      lb.load(g.B, g.ldb, n0, g.N, k0 + TK, ke, t);
+      lb.load(g.B, g.ldb, n0, g.N, k0 + TK, ke, tb);
     }
 #pragma unroll
     for (int kk = 0; kk < TK; kk += 32) {
@@ -336,7 +347,10 @@ __global__ void k_splitsum(const float* part, int S, long long count, float* out
 }
 
 // 64x64 tiles, or 32x32 when the 64x64 grid has fewer than two workgroups
-// per CU (256 CUs).
+// per CU (256 CUs): each step waits for its operands, which only more
+// workgroups hide.  64x32 tiles with 512 workgroups (a quarter less traffic)
+// were slower, 151 against 137 us over the six products that had 1024 of
+// 32x32, and so was a second step of operands on the way (142).
 template <bool TA, bool TB, int EPI>
 hipError_t gemm(const GemmArgs& g, hipStream_t s) {
   const long long big = (long long)((g.N + 63) / 64) * ((g.M + 63) / 64);
@@ -880,27 +894,29 @@ struct nf3d_mlp {
     else mcheck(fwd<EPI_BIAS>(a, s), "layer 3");
   }
 
-  // Forward with the activations kept, Whittle loss, gradients into g.
+  // Forward with the activations kept, Whittle loss, gradients into g.  The
+  // forward products read the transposed weights (k contiguous, as LDS wants
+  // it: 58 -> 38 us at 4096 rows through 1200-256-256-1200); the sums are the same.
   void grad(const __bf16* X, const float* T, int n, hipStream_t s) {
-    GemmArgs a = args(X, n_in, pb + o_w1, nh, n, nh, n_in);
+    GemmArgs a = args(X, n_in, pbt + t_w1, n_in, n, nh, n_in);
     a.bias = p + o_b1;
     a.C = z1;
     a.ldc = nh;
     a.H = h1;
     a.ldh = nh;
-    mcheck(gemm<false, false, EPI_BIAS_GELU>(a, s), "layer 1");
-    a = args(h1, nh, pb + o_w2, nh, n, nh, nh);
+    mcheck(gemm<false, true, EPI_BIAS_GELU>(a, s), "layer 1");
+    a = args(h1, nh, pbt + t_w2, nh, n, nh, nh);
     a.bias = p + o_b2;
     a.C = z2;
     a.ldc = nh;
     a.H = h2;
     a.ldh = nh;
-    mcheck(gemm<false, false, EPI_BIAS_GELU>(a, s), "layer 2");
-    a = args(h2, nh, pb + o_w3, n_out, n, n_out, nh);
+    mcheck(gemm<false, true, EPI_BIAS_GELU>(a, s), "layer 2");
+    a = args(h2, nh, pbt + t_w3, nh, n, n_out, nh);
     a.bias = p + o_b3;
     a.C = y;
     a.ldc = n_out;
-    mcheck(gemm<false, false, EPI_BIAS>(a, s), "layer 3");
+    mcheck(gemm<false, true, EPI_BIAS>(a, s), "layer 3");
     const long long tot = (long long)n * n_out;
     hipLaunchKernelGGL(k_whittle, dim3(blocks(tot, 256)), dim3(256), 0, s, y, T, d3, gf, tot,
                        1.0f / (float)tot, lpart);
