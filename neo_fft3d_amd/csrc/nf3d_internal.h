@@ -58,7 +58,7 @@ struct PlaneJob {
   float sharpen, smin_n, smax_n, dehalo, ht2n, kratio2;
   int use_pattern, use_degrid;
   int pattern_per_block;  // pattern2d / pattern3d hold one [bh][outwidth] pattern per block (learned PSD)
-  // matrix-core DFT (32x32 blocks, per-frame kernel): constant tiles and the
+  // matrix-core DFT (32x32, 48x48, 64x64 blocks): constant tiles and the
   // power-of-two operand scales of the forward and inverse transforms
   const void* dft_tab;
   float dft_sx, dft_sz;
@@ -130,7 +130,7 @@ struct PatternJob {
 // compiled block shape; unsupported shapes return hipErrorInvalidValue.
 // launch_tile runs k_tile and, for the filtering modes, k_seam.
 hipError_t launch_tile(int mode, int bt, int onchip, int mf, int bw, int bh, const TileLaunch& l, hipStream_t s);
-// Block shapes with a matrix-core DFT variant of k_tile (mf = 1).
+// Block shapes with a matrix-core DFT variant of k_tile and k_run (mf = 1).
 bool mfma_dft_supported(int bw, int bh);
 hipError_t launch_pattern(const PatternJob& job, hipStream_t s);
 // Per-region patterns after launch_pattern (which fills sums, and choice if given):
