@@ -23,7 +23,7 @@ struct __attribute__((packed, aligned(4))) Quad {
 // in address order.  The products' own accesses touch 8 to 16 rows at a time,
 // spectral rows of (N/2+1) * 8 bytes that straddle cache lines: in memory
 // those were partial lines, in LDS they are not.  Bound by memory: 32,776
-// blocks of 32x32 forward and back took 157 us, now 132 (278 MB each way; a
+// blocks of 32x32 forward and back took 157 us, now 132 (277 MB each way; a
 // large copy would need 113), 9,001 blocks of 48x48 113 -> 100, of 64x64 241
 // -> 224.  block_in reads all it can before it writes (inverse: 69 -> 65 us);
 // the forward samples come 32 bytes a lane from whole rows and go straight to
