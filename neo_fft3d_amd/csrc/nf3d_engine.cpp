@@ -180,6 +180,8 @@ struct nf3d_engine {
   float2* d_grid = nullptr;
   size_t spec_elems = 0;  // nb * bh * outwidth
   float2* d_ring = nullptr;
+  float2* d_ring2 = nullptr;   // paired runs (RangePlan::paired): bt slots of the other run
+  bool ring2_refused = false;  // no memory for it: unpaired
   int ring_slots = 0;
   std::vector<int> ring_frame;
   std::vector<char> ring_by_run;  // the slot's spectrum came from the frame-loop kernel
@@ -276,6 +278,7 @@ struct nf3d_engine {
     hipFree(d_tab);
     hipFree(d_grid);
     hipFree(d_ring);
+    hipFree(d_ring2);
     hipFree(d_kal_last);
     hipFree(d_kal_sum);
     hipFree(d_seam);
@@ -1048,6 +1051,7 @@ struct nf3d_engine {
   }
 
   // Tiles of a block row in the frame-loop kernel.
+  static constexpr int kPairFrames = 4;  // least frames of a run of a pair (at least bt - 1)
   int run_ntx() const {
     const int bpw = nf3d::run_blocks_per_wg(ep.bw, ep.bh, dft_mode);
     return (nox + bpw - 1) / bpw;
@@ -1090,12 +1094,37 @@ struct nf3d_engine {
     // from its frame: one frame each)
     std::vector<RunLaunch> edges_start, edges;
     // Wiener 3D: the forward transforms of the first window's older frames
-    // that the ring does not hold (none, or one launch)
+    // that the ring does not hold, and those of the first pair's second run
     std::vector<RunLaunch> fwd;
+    // Wiener 3D: launches 2l and 2l + 1 run side by side as two jobs of one
+    // launch (pair_runs), the first in the ring that the run before it left,
+    // the second in the other one, whose older frames are transformed first;
+    // `copy`: the last run ends in d_ring2
+    bool paired = false, copy = false;
+    size_t steps() const { return paired ? launches.size() / 2 : launches.size(); }
   };
 
+  // Forward transforms of frames [k0, k1) into their slots of `ring`.
+  RunLaunch forward_job(const RangePlan& P, int k0, int k1, float2* ring) const {
+    RunLaunch R = run_job();
+    R.J.src_pitch = P.src_pitch;
+    R.J.dst_pitch = P.dst_pitch;
+    for (int k = k0; k < k1; k++) R.src[k - k0] = static_cast<const uint8_t*>(P.src[k]);
+    R.ring = ring;
+    R.spec_elems = (long long)spec_elems;
+    R.m0 = k0;
+    R.nframes = k1 - k0;
+    R.fpw = 1;  // (the frames are independent)
+    return R;
+  }
+  // ... of the older frames of the first window of run j.
+  RunLaunch forward_job(const RangePlan& P, size_t j) const {
+    const RunLaunch& R = P.launches[j];
+    return forward_job(P, R.m0 + P.from, R.m0 + P.to, R.ring);
+  }
+
   RangePlan plan_range(int first, int count, const void* const* src, long long src_pitch, void* const* dst,
-                       long long dst_pitch) {
+                       long long dst_pitch, bool paired) {
     for (int n = first; n < first + count; n++)
       if (n < 0 || n >= frames) fail("frame " + std::to_string(n) + " outside the clip");
     RangePlan P;
@@ -1140,6 +1169,21 @@ struct nf3d_engine {
     // buffers in turn
     const size_t seam_frame = (size_t)4 * Hc * Wc;
     if (!d_seam_run) d_seam_run = dev_alloc<float>(2 * kRunFrames * seam_frame);
+    // two runs side by side (pair_runs): each of some frames, so that the
+    // second one's first window (bt - 1 older frames, transformed once more)
+    // does not cost what the pair gains, and lies within the range
+    const int whole = P.b - P.a + 1, need = (whole + run_frames - 1) / run_frames, even = (need + 1) / 2 * 2;
+    P.paired = paired && P.mode == nf3d::MODE_W3D && whole / even >= kPairFrames && !ring2_refused;
+    if (P.paired && !d_ring2) {
+      void* p = nullptr;
+      if (hipMalloc(&p, spec_elems * ep.bt * sizeof(float2)) == hipSuccess) {
+        d_ring2 = static_cast<float2*>(p);
+      } else {
+        (void)hipGetLastError();
+        ring2_refused = true;
+        P.paired = false;
+      }
+    }
     // the spans of one learned-PSD prediction each (the whole range without
     // a prediction period), each in launches of equal length
     std::vector<std::pair<int, int>> spans;
@@ -1156,7 +1200,7 @@ struct nf3d_engine {
     long long cur = lspan;
     for (const auto& sp : spans) {
       const int total = sp.second - sp.first + 1;
-      const int nl = (total + run_frames - 1) / run_frames;
+      const int nl = P.paired ? even : (total + run_frames - 1) / run_frames;
       for (int jj = 0, m0 = sp.first; jj < nl; jj++, j++) {
         const int nf = total / nl + (jj >= nl - total % nl ? 1 : 0);
         RunLaunch R = run_job();
@@ -1230,23 +1274,28 @@ struct nf3d_engine {
       // the slot holds that frame from that kernel already (a previous call)
       int k0 = P.a + P.from;
       while (k0 < P.a + P.to && ring_frame[k0 % ep.bt] == k0 && ring_by_run[k0 % ep.bt]) k0++;
-      if (k0 < P.a + P.to) {
-        RunLaunch R = run_job();
-        R.J.src_pitch = P.src_pitch;
-        R.J.dst_pitch = P.dst_pitch;
-        for (int k = k0; k < P.a + P.to; k++) R.src[k - k0] = static_cast<const uint8_t*>(P.src[k]);
-        R.ring = d_ring;
-        R.spec_elems = (long long)spec_elems;
-        R.m0 = k0;
-        R.nframes = P.a + P.to - k0;
-        R.fpw = 1;  // (the frames are independent)
-        P.fwd.push_back(R);
+      int start = 0;  // the first run's ring: d_ring, or d_ring2
+      if (P.paired) {
+        // the rings change roles with every pair; with an odd number of pairs
+        // and nothing to keep of d_ring, the first run takes the other one,
+        // so that the last run ends in d_ring
+        const int pairs = (int)P.launches.size() / 2;
+        start = pairs % 2 == 1 && k0 == P.a + P.from ? 1 : 0;
+        for (int j = 0; j < 2 * pairs; j++)
+          P.launches[j].ring = (start + j / 2 + j % 2) % 2 ? d_ring2 : d_ring;
+        P.copy = (start + pairs) % 2 == 1;
+        P.fwd.push_back(forward_job(P, 1));
       }
+      if (k0 < P.a + P.to) P.fwd.push_back(forward_job(P, k0, P.a + P.to, start ? d_ring2 : d_ring));
     }
   }
 
   // Ring bookkeeping after the launch of P.fwd.
   void fwd_launched(const RangePlan& P) {
+    if (P.paired) {  // both rings are about to be written: nothing is known until the epilogue
+      std::fill(ring_frame.begin(), ring_frame.end(), -1);
+      return;
+    }
     for (const RunLaunch& R : P.fwd)
       for (int k = R.m0; k < R.m0 + R.nframes; k++) {
         ring_frame[k % ep.bt] = k;
@@ -1531,6 +1580,28 @@ void learned_predictions(const nf3d_run_item* items, const std::vector<nf3d_engi
   }
 }
 
+// Wiener-3D launches of few tiles: a workgroup filters its tile's frames one
+// after the other, 12 us a frame however empty the chip is (480p, 32x32
+// blocks), so two runs of frames of every plane go side by side where twice
+// the tiles still fit the chip's workgroup slots (three per CU; the second run
+// transforms bt - 1 older frames once more).  480p 32/10, 33 frames 456 -> 323
+// us, 10 frames 158 -> 127; 352x288 64/16, 64 frames 1272 -> 709; with 692 to
+// 748 tiles in a pair 771 -> 597 (720p 48/16, 33 frames), 231 -> 194 (1100x620
+// 32/10, 12 frames) and, where only two workgroups share a CU, 562 -> 459
+// (1340x760 48/16 bt=4, 21 frames), 410 -> 408 at the least (1500x844 64/16
+// bt=5, 12 frames).  More tiles would queue.
+constexpr int kPairTiles = 768;
+bool pair_runs(const nf3d_run_item* items, int n) {
+  if (2 * n > nf3d::RUN_MAX_JOBS) return false;
+  int tiles = 0;
+  for (int i = 0; i < n; i++) {
+    const nf3d_engine* e = items[i].engine;
+    if (e->ep.bt < 2 || e->learned) return false;  // (a learned PSD is predicted per launch)
+    tiles += e->noy * e->run_ntx();
+  }
+  return 2 * tiles <= kPairTiles;
+}
+
 // keep_events: under graph capture, the fork and join events are handed
 // there, to be destroyed after the capture ends, instead of here.
 void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, bool capture = false,
@@ -1538,9 +1609,10 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
   if (!capture)
     for (int i = 0; i < n; i++) items[i].engine->order_before(s);
   std::vector<nf3d_engine::RangePlan> plans(n);
+  const bool paired = pair_runs(items, n);
   for (int i = 0; i < n; i++) {
     const nf3d_run_item& it = items[i];
-    plans[i] = it.engine->plan_range(it.first, it.count, it.src, it.src_stride, it.dst, it.dst_stride);
+    plans[i] = it.engine->plan_range(it.first, it.count, it.src, it.src_stride, it.dst, it.dst_stride, paired);
   }
   // the launches before and after the frame-loop ones, engines of the same
   // shape, sharpen case and transform form (forward transforms: and bt)
@@ -1564,10 +1636,15 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
       }
       size_t nq = 0;
       for (int k : group) nq = std::max(nq, (plans[k].*which).size());
-      for (size_t q = 0; q < nq; q++) {
+      for (size_t q = 0; q < (fwd ? 1 : nq); q++) {
         std::vector<int> members;
+        std::vector<size_t> at;  // index in the member's list (forward transforms: all of them together)
         for (int k : group)
-          if (q < (plans[k].*which).size()) members.push_back(k);
+          for (size_t q1 = q; q1 < (fwd ? nq : q + 1); q1++)
+            if (q1 < (plans[k].*which).size()) {
+              members.push_back(k);
+              at.push_back(q1);
+            }
         for (size_t c0 = 0; c0 < members.size(); c0 += nf3d::RUN_MAX_JOBS) {
           nf3d::RunBatch B{};
           std::vector<std::pair<hipEvent_t, hipEvent_t>> evs;
@@ -1575,7 +1652,7 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
             const int k = members[c];
             nf3d_engine* e = items[k].engine;
             RunLaunch& R = B.job[B.njobs++];
-            R = (plans[k].*which)[q];
+            R = (plans[k].*which)[at[c]];
             R.wg_begin = B.total_wg;
             B.total_wg += R.ntiles * R.nframes;
             B.max_hc = std::max(B.max_hc, e->Hc);
@@ -1649,11 +1726,29 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
     const hipStream_t gs = groups.size() > 1 ? e0->stream : s;
     if (gs != s) check(hipStreamWaitEvent(gs, fork, 0), "hipStreamWaitEvent");
     size_t nl = 0;
-    for (int k : group) nl = std::max(nl, plans[k].launches.size());
+    for (int k : group) nl = std::max(nl, plans[k].steps());
     for (size_t l = 0; l < nl; l++) {
       std::vector<int> members;
-      for (int k : group)
-        if (l < plans[k].launches.size()) members.push_back(k);
+      std::vector<size_t> at;  // launch of the member's plan
+      nf3d::RunBatch F{};      // first windows of the pairs' second runs (of the first pair: with P.fwd)
+      for (int k : group) {
+        const nf3d_engine::RangePlan& P = plans[k];
+        if (l >= P.steps()) continue;
+        members.push_back(k);
+        at.push_back(P.paired ? 2 * l : l);
+        if (!P.paired) continue;
+        members.push_back(k);
+        at.push_back(2 * l + 1);
+        if (l == 0) continue;
+        RunLaunch& R = F.job[F.njobs++];
+        R = items[k].engine->forward_job(P, 2 * l + 1);
+        R.wg_begin = F.total_wg;
+        F.total_wg += R.ntiles * R.nframes;
+        F.max_frames = std::max(F.max_frames, R.nframes);
+      }
+      if (F.njobs)
+        check(nf3d::launch_run(nf3d::MODE_FWD, e0->ep.bt, nf3d::SHP_NONE, e0->dft_mode, e0->ep.bw, e0->ep.bh, F, gs),
+              "frame-loop forward transforms");
       for (size_t c0 = 0; c0 < members.size(); c0 += nf3d::RUN_MAX_JOBS) {
         nf3d::RunBatch B{};
         std::vector<std::pair<hipEvent_t, hipEvent_t>> evs;
@@ -1661,15 +1756,19 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
           const int k = members[c];
           nf3d_engine* e = items[k].engine;
           RunLaunch& R = B.job[B.njobs++];
-          R = plans[k].launches[l];
+          R = plans[k].launches[at[c]];
           R.wg_begin = B.total_wg;
           B.total_wg += R.ntiles * ((R.nframes + R.fpw - 1) / R.fpw);
           B.max_hc = std::max(B.max_hc, e->Hc);
           B.max_frames = std::max(B.max_frames, R.nframes);
         }
         learned_predictions(items, plans, members, c0, B, plans[i].mode, l, gs);
-        for (int c = 0; c < B.njobs; c++)
-          evs.push_back(items[members[c0 + c]].engine->timer(timed, B.job[c].nframes, gs));
+        for (int c = 0; c < B.njobs; c++) {
+          const nf3d_engine::RangePlan& P = plans[members[c0 + c]];
+          if (P.paired && at[c0 + c] % 2 == 1) continue;  // timed with the run beside it
+          evs.push_back(items[members[c0 + c]].engine->timer(
+              timed, B.job[c].nframes + (P.paired ? B.job[c + 1].nframes : 0), gs));
+        }
         // the seam pass follows on the same stream: run beside the next
         // launch it takes issue slots the latency-bound k_run needs more
         check(nf3d::launch_run(plans[i].mode, e0->ep.bt, plans[i].shp, e0->dft_mode, e0->ep.bw, e0->ep.bh, B, gs),
@@ -1678,6 +1777,12 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
         for (auto& ev : evs)
           if (ev.second) check(hipEventRecord(ev.second, gs), "hipEventRecord");
       }
+    }
+    for (int k : group) {
+      const nf3d_engine* e = items[k].engine;
+      if (plans[k].copy)
+        check(hipMemcpyAsync(e->d_ring, e->d_ring2, sizeof(float2) * e->spec_elems * e->ep.bt, hipMemcpyDeviceToDevice, gs),
+              "spectra of the last run");
     }
     if (gs != s) {
       hipEvent_t j = nullptr;
@@ -2092,7 +2197,7 @@ int capture_batch(const nf3d_run_item* items, int n, void* stream, nf3d_graph** 
       }
       // buffers the launches use, allocated outside the capture
       e->plan_range(items[i].first, items[i].count, items[i].src, items[i].src_stride, items[i].dst,
-                    items[i].dst_stride);
+                    items[i].dst_stride, pair_runs(items, n));
     }
     // no profiling events inside the graph
     std::vector<bool> prof(n);
