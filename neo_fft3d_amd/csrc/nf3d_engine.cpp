@@ -963,7 +963,20 @@ struct nf3d_engine {
     use_learned(J);
   }
 
+  // Cut short (a missing frame, no memory), it forgets the ring slots that it
+  // claimed: nothing may have been computed there.
   void run(int n, const Call& c, uint8_t* dst, long long dst_pitch) {
+    const uint64_t before = tick;
+    try {
+      run_frame(n, c, dst, dst_pitch);
+    } catch (...) {
+      for (int i = 0; i < ring_slots; i++)
+        if (ring_tick[i] > before) ring_frame[i] = -1;
+      throw;
+    }
+  }
+
+  void run_frame(int n, const Call& c, uint8_t* dst, long long dst_pitch) {
     check(hipSetDevice(device), "hipSetDevice");
     if (ep.pfactor != 0 && ep.pshow) {
       run_pshow(n, c, dst, dst_pitch);
