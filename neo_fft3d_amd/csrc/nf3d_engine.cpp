@@ -61,13 +61,14 @@ void check(hipError_t e, const char* what) {
   }
 }
 
-void copy_err(char* err, size_t len, const std::string& m) {
+void copy_err(char* err, size_t len, const char* m) {
   if (err && len) {
-    size_t n = std::min(len - 1, m.size());
-    memcpy(err, m.data(), n);
+    size_t n = std::min(len - 1, strlen(m));
+    memcpy(err, m, n);
     err[n] = 0;
   }
 }
+void copy_err(char* err, size_t len, const std::string& m) { copy_err(err, len, m.c_str()); }
 
 // Launch tuning of the frame-loop path (results do not depend on it, except
 // with a learned PSD, which is predicted once per launch: table entries do
@@ -1377,24 +1378,28 @@ int nf3d_engine_frame_begin(nf3d_engine* e, int n, const nf3d_frame_ref* frames,
   try {
     e->last_end = -1;
     e->frame_begin(n, frames, nframes, dst, dst_stride);
+    lock.release();  // nf3d_engine_frame_end unlocks
+    return 0;
   } catch (const Failure& f) {
-    (void)hipStreamSynchronize(e->stream);  // the staging buffers are free for the next call
     copy_err(err, errlen, f.msg);
-    return -1;
+  } catch (const std::exception& x) {
+    copy_err(err, errlen, x.what());
   }
-  lock.release();  // nf3d_engine_frame_end unlocks
-  return 0;
+  (void)hipStreamSynchronize(e->stream);  // the staging buffers are free for the next call
+  return -1;
 }
 
 int nf3d_engine_frame_end(nf3d_engine* e, char* err, size_t errlen) {
   std::unique_lock<std::mutex> lock(e->mu, std::adopt_lock);
   try {
     e->frame_end();
+    return 0;
   } catch (const Failure& f) {
     copy_err(err, errlen, f.msg);
-    return -1;
+  } catch (const std::exception& x) {
+    copy_err(err, errlen, x.what());
   }
-  return 0;
+  return -1;
 }
 
 // ---------------------------------------------------------------- C ABI

@@ -319,37 +319,51 @@ int nf3d_filter_get_frame(nf3d_filter* f, int n, const nf3d_frame_planes* frames
   const nf3d_frame_planes* cur = nullptr;
   for (int i = 0; i < nframes; i++)
     if (frames[i].n == n) cur = &frames[i];
-  if (!cur) {
-    put_err(err, errlen, "frame " + std::to_string(n) + " was not provided");
+  try {
+    if (!cur) {
+      put_err(err, errlen, "frame " + std::to_string(n) + " was not provided");
+      return -1;
+    }
+    std::vector<nf3d_frame_ref> refs(nframes);
+    // every plane is queued (its staging copies overlap the planes before on
+    // the GPU), then each is waited for and copied out; a plane begun is ended
+    // however the others fare
+    struct Begun {
+      nf3d_engine* e[4];
+      int n = 0, at = 0;
+      bool end(char* msg, size_t len) { return nf3d_engine_frame_end(e[at++], msg, len) == 0; }
+      ~Begun() {
+        while (at < n) end(nullptr, 0);
+      }
+    } begun;
+    for (int pl = 0; pl < f->fmt.num_planes; pl++) {
+      int w, h;
+      f->plane_dims(pl, w, h);
+      auto copy_src = [&]() {
+        const uint8_t* s = static_cast<const uint8_t*>(cur->data[pl]);
+        uint8_t* d = static_cast<uint8_t*>(dst[pl]);
+        for (int y = 0; y < h; y++)
+          memcpy(d + (size_t)y * dst_stride[pl], s + (size_t)y * cur->stride[pl], (size_t)w * f->bps);
+      };
+      if (f->process[pl] == 3) {
+        if (f->crop) copy_src();  // borders keep the source (src/fft3d.hpp:315-351)
+        for (int i = 0; i < nframes; i++)
+          refs[i] = nf3d_frame_ref{frames[i].n, frames[i].data[pl], frames[i].stride[pl]};
+        if (nf3d_engine_frame_begin(f->eng[pl], n, refs.data(), nframes, dst[pl], dst_stride[pl], err, errlen) != 0)
+          return -1;
+        begun.e[begun.n++] = f->eng[pl];
+      } else if (f->process[pl] == 2) {
+        copy_src();
+      }
+    }
+    bool ok = true;
+    while (begun.at < begun.n)
+      if (!begun.end(ok ? err : nullptr, ok ? errlen : 0)) ok = false;
+    if (!ok) return -1;
+  } catch (const std::exception& x) {
+    put_err(err, errlen, x.what());
     return -1;
   }
-  std::vector<nf3d_frame_ref> refs(nframes);
-  // every plane is queued (its staging copies overlap the planes before on
-  // the GPU), then each is waited for and copied out
-  nf3d_engine* begun[4];
-  int nbegun = 0;
-  bool ok = true;
-  for (int pl = 0; pl < f->fmt.num_planes && ok; pl++) {
-    int w, h;
-    f->plane_dims(pl, w, h);
-    auto copy_src = [&]() {
-      const uint8_t* s = static_cast<const uint8_t*>(cur->data[pl]);
-      uint8_t* d = static_cast<uint8_t*>(dst[pl]);
-      for (int y = 0; y < h; y++)
-        memcpy(d + (size_t)y * dst_stride[pl], s + (size_t)y * cur->stride[pl], (size_t)w * f->bps);
-    };
-    if (f->process[pl] == 3) {
-      if (f->crop) copy_src();  // borders keep the source (src/fft3d.hpp:315-351)
-      for (int i = 0; i < nframes; i++) refs[i] = nf3d_frame_ref{frames[i].n, frames[i].data[pl], frames[i].stride[pl]};
-      ok = nf3d_engine_frame_begin(f->eng[pl], n, refs.data(), nframes, dst[pl], dst_stride[pl], err, errlen) == 0;
-      if (ok) begun[nbegun++] = f->eng[pl];
-    } else if (f->process[pl] == 2) {
-      copy_src();
-    }
-  }
-  for (int i = 0; i < nbegun; i++)
-    if (nf3d_engine_frame_end(begun[i], ok ? err : nullptr, ok ? errlen : 0) != 0) ok = false;
-  if (!ok) return -1;
   f->pattern_pending = false;
   return 0;
 }

@@ -222,11 +222,62 @@ void missing_frame() {
   }
 }
 
+// A frame of a 4:2:0 filter (bt = 1).
+struct Frame {
+  nf3d_filter* f = nullptr;
+  std::vector<uint8_t> in, out;
+  nf3d_frame_planes fr{};
+  void* dst[4] = {};
+  int stride[4] = {W, W / 2, W / 2, 0};
+  Frame() : in(W * H * 3 / 2), out(in.size()) {
+    nf3d_format fmt{};
+    fmt.color_family = 1;
+    fmt.bits_per_sample = 8;
+    fmt.ssw = fmt.ssh = 1;
+    fmt.num_planes = 3;
+    char err[256] = {0};
+    CHECK(nf3d_filter_create("bt=1;bw=16;bh=16;ow=4;oh=4", &fmt, W, H, FRAMES, &f, err, sizeof err) == 0);
+    for (size_t i = 0; i < in.size(); i++) in[i] = (uint8_t)(i * 7 + (i >> 8));
+    size_t o = 0;
+    for (int p = 0; p < 3; p++) {
+      fr.data[p] = &in[o];
+      fr.stride[p] = stride[p];
+      dst[p] = &out[o];
+      o += (size_t)stride[p] * (p ? H / 2 : H);
+    }
+  }
+  int get(std::string* msg = nullptr) {
+    char err[256] = {0};
+    std::fill(out.begin(), out.end(), 0);
+    const int rc = nf3d_filter_get_frame(f, 0, &fr, 1, dst, stride, err, sizeof err);
+    if (msg) *msg = err;
+    return rc;
+  }
+};
+
+// An exception in the pinned allocation `at` of a frame, so while one of its
+// planes is queued: an error, and every plane's engine is free again (a lock
+// left behind would stop the next call for good).
+void frame_throws() {
+  for (int at = 0; at < 6; at++) {
+    Frame F;
+    std::string msg;
+    pinned_throw = at;
+    CHECK(F.get(&msg) == -1);
+    CHECK(!msg.empty());
+    pinned_throw = -1;
+    CHECK(F.get() == 0);
+    CHECK(F.out == F.in);
+    nf3d_filter_destroy(F.f);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "missing_frame") missing_frame();
+  else if (name == "frame_throws") frame_throws();
   else return 2;
   return 0;
 }
