@@ -133,10 +133,12 @@ T* dev_alloc(size_t count) {
   return static_cast<T*>(p);
 }
 
+// Page-locked memory, or null where the system grants none.
 uint8_t* pinned_alloc(size_t bytes) {
   void* p = nullptr;
-  check(hipHostMalloc(&p, std::max<size_t>(bytes, 1), hipHostMallocDefault), "hipHostMalloc");
-  return static_cast<uint8_t*>(p);
+  if (hipHostMalloc(&p, std::max<size_t>(bytes, 1), hipHostMallocDefault) == hipSuccess) return static_cast<uint8_t*>(p);
+  (void)hipGetLastError();
+  return nullptr;
 }
 
 // What the runtime knows of p: memory of ordinary allocations (pageable) is
@@ -204,8 +206,9 @@ struct nf3d_engine {
   size_t stage_pitch = 0;
   int stage_next = 0;
   uint8_t* d_dst = nullptr;
-  // pinned staging of the pageable planes of a host-fed frame: an upload
-  // buffer for each plane of one call, and the output's
+  // pinned staging of the pageable planes of a host-fed frame, kept until the
+  // engine goes: an upload buffer for each plane that one call brings (bt, and
+  // the pattern's frame, at most; one in order), and the output's
   std::vector<uint8_t*> h_up;
   size_t h_up_used = 0;
   uint8_t* h_down = nullptr;
@@ -652,6 +655,17 @@ struct nf3d_engine {
     return nullptr;
   }
 
+  // The next upload buffer of this call, or null.
+  uint8_t* upload_staging() {
+    if (h_up_used == h_up.size()) {
+      h_up.reserve(h_up.size() + 1);
+      uint8_t* p = pinned_alloc(stage_pitch * frameheight);
+      if (!p) return nullptr;
+      h_up.push_back(p);
+    }
+    return h_up[h_up_used++];
+  }
+
   Src source(const Call& c, int k) {
     const nf3d_frame_ref* fr = find(c, k);
     if (!fr || !fr->data) fail("frame " + std::to_string(k) + " was not provided");
@@ -668,19 +682,19 @@ struct nf3d_engine {
     stage_next = (stage_next + 1) % (int)d_stage.size();
     stage_frame[slot] = k;
     const size_t row = (size_t)framewidth * pix;
-    if (memory_type(fr->data) != hipMemoryTypeUnregistered) {
+    const bool pageable = memory_type(fr->data) == hipMemoryTypeUnregistered;
+    if (pageable && fr->stride < (long long)row) check(hipErrorInvalidPitchValue, "upload");
+    // pageable memory: through pinned staging laid out like the device slot,
+    // in chunks that go up while the next one is copied (the runtime's own 2D
+    // copy of pageable rows, taken where no memory is left to pin, moved 0.2
+    // GB/s: 11 ms for each plane of a 1920x1080 frame and way)
+    uint8_t* h = pageable ? upload_staging() : nullptr;
+    if (!h) {
       check(hipMemcpy2DAsync(d_stage[slot], stage_pitch, fr->data, fr->stride, row, frameheight, hipMemcpyHostToDevice,
                              c.s),
             "upload");
       return Src{d_stage[slot], (long long)stage_pitch};
     }
-    // pageable memory: through pinned staging laid out like the device slot,
-    // in chunks that go up while the next one is copied (the runtime's own 2D
-    // copy of pageable rows moved 0.2 GB/s: 11 ms for each plane of a
-    // 1920x1080 frame and way)
-    if (fr->stride < (long long)row) check(hipErrorInvalidPitchValue, "upload");
-    if (h_up_used == h_up.size()) h_up.push_back(pinned_alloc(stage_pitch * frameheight));
-    uint8_t* h = h_up[h_up_used++];
     const int step = std::max<int>(1, (int)(kUploadChunk / stage_pitch));
     for (int y = 0; y < frameheight; y += step) {
       const int rows = std::min(step, frameheight - y);
@@ -1350,14 +1364,15 @@ struct nf3d_engine {
     run(n, c, d_dst, (long long)dpitch);
     uint8_t* from = d_dst + (size_t)tc * dpitch;
     uint8_t* to = static_cast<uint8_t*>(dst) + (size_t)tc * dst_stride + (size_t)lc * pix;
-    if (memory_type(dst) != hipMemoryTypeUnregistered) {
+    const bool pageable = memory_type(dst) == hipMemoryTypeUnregistered;
+    if (pageable && !dst) check(hipErrorInvalidValue, "download");
+    if (pageable && dst_stride < (long long)row) check(hipErrorInvalidPitchValue, "download");
+    if (pageable && !h_down) h_down = pinned_alloc(dpitch * frameheight);
+    if (!pageable || !h_down) {
       check(hipMemcpy2DAsync(to, dst_stride, from + (size_t)lc * pix, dpitch, row, Hc, hipMemcpyDeviceToHost, stream),
             "download");
       return;
     }
-    if (!dst) check(hipErrorInvalidValue, "download");
-    if (dst_stride < (long long)row) check(hipErrorInvalidPitchValue, "download");
-    if (!h_down) h_down = pinned_alloc(dpitch * frameheight);
     check(hipMemcpyAsync(h_down, from, dpitch * Hc, hipMemcpyDeviceToHost, stream), "download");
     out_dst = to;
     out_stride = dst_stride;

@@ -272,12 +272,29 @@ void frame_throws() {
   }
 }
 
+// Page-locked memory refused: the frame comes all the same, then and after.
+void pinned_refused() {
+  for (int at = 0; at <= 6; at++) {
+    Frame F;
+    pinned_left = at;
+    CHECK(F.get() == 0);
+    CHECK(F.out == F.in);
+    CHECK(F.get() == 0);
+    CHECK(F.out == F.in);
+    pinned_left = -1;
+    CHECK(F.get() == 0);
+    CHECK(F.out == F.in);
+    nf3d_filter_destroy(F.f);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "missing_frame") missing_frame();
   else if (name == "frame_throws") frame_throws();
+  else if (name == "pinned_refused") pinned_refused();
   else return 2;
   return 0;
 }
