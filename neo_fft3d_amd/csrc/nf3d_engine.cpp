@@ -225,7 +225,7 @@ struct nf3d_engine {
       if (ev) (void)hipEventDestroy(ev);
     }
   };
-  std::shared_ptr<Mark> own_mark, done;  // (done: this engine's or its batch's first engine's)
+  std::shared_ptr<Mark> own_mark[2], done;  // (done: this engine's or its batch's first engine's)
   hipStream_t done_stream = nullptr;
   // opt-in HIP-event timing of the main spectral kernel of each frame
   bool profiling = false;
@@ -728,18 +728,24 @@ struct nf3d_engine {
     if (done_stream && done_stream != s) check(hipStreamWaitEvent(s, done->ev, 0), "hipStreamWaitEvent");
   }
   // ... and marks its own end: one event for all engines of a batch (an event
-  // each cost 4 us of the stream's time).  The event is the first engine's,
-  // shared with the others; when that engine records it again for a later call
-  // of its own, that call has come after the batch's work, so a wait for the
-  // event still covers it.
+  // each cost 4 us of the stream's time), the first engine's, shared with the
+  // others.  An event that another engine still holds is not recorded again --
+  // that engine's next call would wait for whatever this one did alone -- but
+  // the engine's other one is, free in a loop of batches (another engine only
+  // ever lets go of a mark by itself, so one seen unshared stays so), or a new
+  // one.
   void order_after(hipStream_t s) {
-    if (!own_mark) {
-      auto m = std::make_shared<Mark>();
-      check(hipEventCreateWithFlags(&m->ev, hipEventDisableTiming), "hipEventCreate");
-      own_mark = m;
+    std::shared_ptr<Mark>* m = nullptr;
+    for (auto& o : own_mark)
+      if (!m && (!o || o.use_count() == (o == done ? 2 : 1))) m = &o;
+    if (!m) (m = &own_mark[0])->reset();
+    if (!*m) {
+      auto f = std::make_shared<Mark>();
+      check(hipEventCreateWithFlags(&f->ev, hipEventDisableTiming), "hipEventCreate");
+      *m = f;
     }
-    check(hipEventRecord(own_mark->ev, s), "hipEventRecord");
-    done = own_mark;
+    check(hipEventRecord((*m)->ev, s), "hipEventRecord");
+    done = *m;
     done_stream = s;
   }
   void order_after(hipStream_t s, const nf3d_engine& first) {

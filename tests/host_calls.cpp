@@ -201,6 +201,20 @@ nf3d_engine* engine(int bt, int w = W, int h = H) {
   return e;
 }
 
+// A call of frames [first, first + count) of every engine on stream s.
+void batch(const std::vector<nf3d_engine*>& es, Planes& P, int first, int count, hipStream_t s) {
+  std::vector<nf3d_run_item> it;
+  for (nf3d_engine* e : es) it.push_back(nf3d_run_item{e, first, count, P.src.data(), W, P.dst.data(), W});
+  char err[256] = {0};
+  CHECK(nf3d_run_device_batch(it.data(), (int)it.size(), s, err, sizeof err) == 0);
+}
+
+bool waited_for(hipStream_t on, hipStream_t record) {
+  for (const Wait& w : waits)
+    if (w.on == on && w.record == record) return true;
+  return false;
+}
+
 // A call that lacks a frame of its window leaves no frame recorded in the
 // ring that nothing transformed.
 void missing_frame() {
@@ -288,6 +302,40 @@ void pinned_refused() {
   }
 }
 
+// Engines that met in one batch and part: each waits for the batch, not for
+// what the others did later; no events are made once the calls repeat; an
+// engine's mark outlives it.
+void engines_part() {
+  Planes P(W, H);
+  nf3d_engine *a = engine(1), *b = engine(1), *c = engine(1);
+  batch({a, b, c}, P, 0, 2, stream(1));
+  batch({a}, P, 2, 2, stream(2));
+  CHECK(waited_for(stream(2), stream(1)));
+  batch({b}, P, 2, 2, stream(3));
+  CHECK(waited_for(stream(3), stream(1)) && !waited_for(stream(3), stream(2)));
+  synced.clear();
+  nf3d_engine_sync(c);
+  CHECK(synced == std::vector<hipStream_t>{stream(1)});
+  // together again on a fourth stream: the batch waits for both
+  batch({a, b}, P, 4, 2, stream(4));
+  CHECK(waited_for(stream(4), stream(2)) && waited_for(stream(4), stream(3)));
+  for (int k = 0; k < 4; k++) batch({a, b, c}, P, 6, 2, stream(5));
+  const int made = events_made;
+  for (int k = 0; k < 40; k++) batch({a, b, c}, P, 6, 2, stream(5));
+  for (int k = 0; k < 40; k++) {
+    batch({a, b, c}, P, 6, 2, stream(5));
+    batch({a}, P, 8, 2, stream(6));
+  }
+  CHECK(events_made <= made + 1);
+  nf3d_engine_destroy(a);
+  waits.clear();
+  batch({b, c}, P, 8, 2, stream(7));
+  CHECK(waited_for(stream(7), stream(5)));
+  nf3d_engine_destroy(b);
+  nf3d_engine_sync(c);
+  nf3d_engine_destroy(c);
+  CHECK(events.empty());
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -295,6 +343,7 @@ int main(int argc, char** argv) {
   if (name == "missing_frame") missing_frame();
   else if (name == "frame_throws") frame_throws();
   else if (name == "pinned_refused") pinned_refused();
+  else if (name == "engines_part") engines_part();
   else return 2;
   return 0;
 }
