@@ -166,7 +166,7 @@ void copy_rows(uint8_t* dst, size_t dpitch, const uint8_t* src, size_t spitch, s
 struct nf3d_engine {
   nf3d_params ep{};  // scaled copy, as FFT3DEngine keeps it
   nf3d_format fmt{};
-  int plane = 0, chroma = 0, frames = 0, device = 0;
+  int plane = 0, chroma = 0, frames = 0, device = 0, compute_units = 0;
   int framewidth = 0, frameheight = 0, lc = 0, tc = 0, rc = 0, bc = 0, Wc = 0, Hc = 0;
   int nox = 0, noy = 0, nb = 0, outwidth = 0, mirw = 0, mirh = 0, pix = 1;
   float norm = 0, sigma2d = 0, smin_n = 0, smax_n = 0, ht2n = 0;
@@ -549,6 +549,7 @@ struct nf3d_engine {
     build_grid();
 
     check(hipGetDevice(&device), "hipGetDevice");
+    check(hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, device), "hipDeviceGetAttribute");
     check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
     upload_tables();
     spec_elems = (size_t)nb * bh * outwidth;
@@ -1085,7 +1086,6 @@ struct nf3d_engine {
   }
 
   // Tiles of a block row in the frame-loop kernel.
-  static constexpr int kPairFrames = 4;  // least frames of a run of a pair (at least bt - 1)
   int run_ntx() const {
     const int bpw = nf3d::run_blocks_per_wg(ep.bw, ep.bh, dft_mode);
     return (nox + bpw - 1) / bpw;
@@ -1158,7 +1158,7 @@ struct nf3d_engine {
   }
 
   RangePlan plan_range(int first, int count, const void* const* src, long long src_pitch, void* const* dst,
-                       long long dst_pitch, bool paired) {
+                       long long dst_pitch, int pair_frames) {
     for (int n = first; n < first + count; n++)
       if (n < 0 || n >= frames) fail("frame " + std::to_string(n) + " outside the clip");
     RangePlan P;
@@ -1203,11 +1203,11 @@ struct nf3d_engine {
     // buffers in turn
     const size_t seam_frame = (size_t)4 * Hc * Wc;
     if (!d_seam_run) d_seam_run = dev_alloc<float>(2 * kRunFrames * seam_frame);
-    // two runs side by side (pair_runs): each of some frames, so that the
-    // second one's first window (bt - 1 older frames, transformed once more)
-    // does not cost what the pair gains, and lies within the range
+    // two runs side by side (pair_runs): each of some frames (0: none), so that
+    // the second one's first window (bt - 1 older frames, transformed once
+    // more) does not cost what the pair gains, and lies within the range
     const int whole = P.b - P.a + 1, need = (whole + run_frames - 1) / run_frames, even = (need + 1) / 2 * 2;
-    P.paired = paired && P.mode == nf3d::MODE_W3D && whole / even >= kPairFrames && !ring2_refused;
+    P.paired = pair_frames > 0 && P.mode == nf3d::MODE_W3D && whole / even >= pair_frames && !ring2_refused;
     if (P.paired && !d_ring2) {
       void* p = nullptr;
       if (hipMalloc(&p, spec_elems * ep.bt * sizeof(float2)) == hipSuccess) {
@@ -1627,18 +1627,29 @@ void learned_predictions(const nf3d_run_item* items, const std::vector<nf3d_engi
 // us, 10 frames 158 -> 127; 352x288 64/16, 64 frames 1272 -> 709; with 692 to
 // 748 tiles in a pair 771 -> 597 (720p 48/16, 33 frames), 231 -> 194 (1100x620
 // 32/10, 12 frames) and, where only two workgroups share a CU, 562 -> 459
-// (1340x760 48/16 bt=4, 21 frames), 410 -> 408 at the least (1500x844 64/16
-// bt=5, 12 frames).  More tiles would queue.
-constexpr int kPairTiles = 768;
-bool pair_runs(const nf3d_run_item* items, int n) {
-  if (2 * n > nf3d::RUN_MAX_JOBS) return false;
+// (1340x760 48/16 bt=4, 21 frames).  More tiles would queue.
+// Returns the least frames of a run of a pair, or 0 for none: four, but six
+// where the pair does not fit two workgroups per CU (which is what these
+// variants' registers allow) and the four frames of bt = 5 are transformed
+// again: in 768 workgroups of 48 rows, 8 whole windows 325 us unpaired and 334
+// in a pair, 10 376 and 381, but 12 437 and 431, 16 546 and 525.  At bt <= 4
+// (1.02x at 8 frames) and in blocks of up to 32 rows (1.14x at 8 frames) four
+// gain everywhere.  Clips on streams of their own, 1 to 8 of them, lose nothing
+// either: 480p bt=5 4 clips 595 and 595 us, 720p 8 clips 3936 and 3965.
+constexpr int kPairPerCu = 3;
+int pair_runs(const nf3d_run_item* items, int n) {
+  if (2 * n > nf3d::RUN_MAX_JOBS) return 0;
   int tiles = 0;
+  bool tall = false;
   for (int i = 0; i < n; i++) {
     const nf3d_engine* e = items[i].engine;
-    if (e->ep.bt < 2 || e->learned) return false;  // (a learned PSD is predicted per launch)
+    if (e->ep.bt < 2 || e->learned) return 0;  // (a learned PSD is predicted per launch)
     tiles += e->noy * e->run_ntx();
+    tall = tall || (e->ep.bt == 5 && e->ep.bh >= 48);
   }
-  return 2 * tiles <= kPairTiles;
+  const int cus = items[0].engine->compute_units;
+  if (2 * tiles > kPairPerCu * cus) return 0;
+  return tall && 2 * tiles > 2 * cus ? 6 : 4;
 }
 
 // keep_events: under graph capture, the fork and join events are handed
@@ -1648,10 +1659,10 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
   if (!capture)
     for (int i = 0; i < n; i++) items[i].engine->order_before(s);
   std::vector<nf3d_engine::RangePlan> plans(n);
-  const bool paired = pair_runs(items, n);
+  const int pair_frames = pair_runs(items, n);
   for (int i = 0; i < n; i++) {
     const nf3d_run_item& it = items[i];
-    plans[i] = it.engine->plan_range(it.first, it.count, it.src, it.src_stride, it.dst, it.dst_stride, paired);
+    plans[i] = it.engine->plan_range(it.first, it.count, it.src, it.src_stride, it.dst, it.dst_stride, pair_frames);
   }
   // the launches before and after the frame-loop ones, engines of the same
   // shape, sharpen case and transform form (forward transforms: and bt)

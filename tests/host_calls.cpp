@@ -41,7 +41,7 @@ struct Wait {
 };
 std::vector<Wait> waits;
 std::vector<hipStream_t> synced;        // streams of the events waited for on the host
-std::vector<int> run_jobs;              // jobs of each frame-loop launch
+std::vector<int> run_jobs;              // jobs of each Wiener-3D launch
 char handles[4096];
 int next_handle = 1;
 template <class T>
@@ -151,8 +151,8 @@ hipError_t launch_tile(int, int, int, int, int, int, const TileLaunch& l, hipStr
     for (int y = 0; y < J.Hc; y++) memcpy(J.dst + y * J.dst_pitch, J.src + y * J.src_pitch, (size_t)J.Wc * J.pix);
   return hipSuccess;
 }
-hipError_t launch_run(int, int, int, int, int, int, const RunBatch& b, hipStream_t) {
-  run_jobs.push_back(b.njobs);
+hipError_t launch_run(int mode, int, int, int, int, int, const RunBatch& b, hipStream_t) {
+  if (mode == MODE_W3D) run_jobs.push_back(b.njobs);
   return hipSuccess;
 }
 hipError_t launch_seam_run(int, int, int, const RunBatch&, hipStream_t) { return hipSuccess; }
@@ -186,18 +186,18 @@ struct Planes {
   }
 };
 
-nf3d_engine* engine(int bt, int w = W, int h = H) {
+nf3d_engine* engine(int bt, int block = 16) {
   nf3d_params prm;
   nf3d_params_defaults(&prm, 2.0f);
   prm.bt = bt;
-  prm.bw = prm.bh = 16;
-  prm.ow = prm.oh = 4;
+  prm.bw = prm.bh = block;
+  prm.ow = prm.oh = block / 4;
   nf3d_format fmt{};
   fmt.bits_per_sample = 8;
   fmt.num_planes = 1;
   nf3d_engine* e = nullptr;
   char err[256] = {0};
-  CHECK(nf3d_engine_create(&prm, &fmt, w, h, FRAMES, 0, &e, err, sizeof err) == 0);
+  CHECK(nf3d_engine_create(&prm, &fmt, W, H, FRAMES, 0, &e, err, sizeof err) == 0);
   return e;
 }
 
@@ -336,6 +336,33 @@ void engines_part() {
   nf3d_engine_destroy(c);
   CHECK(events.empty());
 }
+
+// Where Wiener-3D runs go in pairs: twice the tiles on the device's three
+// workgroups per CU, and runs of four frames, or, past two per CU, of six in
+// blocks of 48 rows with bt = 5.
+void pairs() {
+  Planes P(W, H);
+  for (int block : {16, 32, 48}) {
+    for (int bt : {2, 3, 5}) {
+      int geo[7];
+      nf3d_engine* e = engine(bt, block);
+      nf3d_engine_geometry(e, geo);
+      nf3d_engine_destroy(e);
+      const int per = nf3d::tile_blocks_per_wg(block, block), wgs = 2 * geo[1] * ((geo[0] + per - 1) / per);
+      for (int cus : {(wgs - 1) / 3, (wgs + 2) / 3, (wgs - 1) / 2, (wgs + 1) / 2}) {
+        compute_units = cus;
+        const int least = wgs > 3 * cus ? FRAMES : bt == 5 && block == 48 && wgs > 2 * cus ? 6 : 4;
+        e = engine(bt, block);
+        for (int whole : {7, 8, 10, 11, 12, 15}) {
+          run_jobs.clear();
+          batch({e}, P, bt / 2, whole, stream(1));
+          CHECK(run_jobs == std::vector<int>{whole >= 2 * least ? 2 : 1});
+        }
+        nf3d_engine_destroy(e);
+      }
+    }
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -344,6 +371,7 @@ int main(int argc, char** argv) {
   else if (name == "frame_throws") frame_throws();
   else if (name == "pinned_refused") pinned_refused();
   else if (name == "engines_part") engines_part();
+  else if (name == "pairs") pairs();
   else return 2;
   return 0;
 }
