@@ -1103,6 +1103,11 @@ struct nf3d_engine {
     if (ep.sharpen == 0.0f && ep.dehalo == 0.0f) return nf3d::SHP_NONE;
     return ep.dehalo == 0.0f ? nf3d::SHP_SHARPEN : nf3d::SHP_GENERAL;
   }
+  // Whether ranges of both engines share frame-loop launches (bt gives the mode).
+  bool same_launch(const nf3d_engine& o) const {
+    return ep.bw == o.ep.bw && ep.bh == o.ep.bh && ep.bt == o.ep.bt && shp_kind() == o.shp_kind() &&
+           dft_mode == o.dft_mode;
+  }
 
   // Plan of a device range: frames [first, first + count) of a device-resident
   // clip, in order.  The frames whose filter window is whole (every frame for
@@ -1636,14 +1641,19 @@ void learned_predictions(const nf3d_run_item* items, const std::vector<nf3d_engi
 // (1.02x at 8 frames) and in blocks of up to 32 rows (1.14x at 8 frames) four
 // gain everywhere.  Clips on streams of their own, 1 to 8 of them, lose nothing
 // either: 480p bt=5 4 clips 595 and 595 us, 720p 8 clips 3936 and 3965.
+// Under capture only batches of one launch group pair: a captured batch of two
+// block shapes, its groups parallel branches of the graph with pairs in them,
+// ended in a segmentation fault in the replay's launch on the host, whose
+// cause is not known; without pairs such graphs are what they were.
 constexpr int kPairPerCu = 3;
-int pair_runs(const nf3d_run_item* items, int n) {
+int pair_runs(const nf3d_run_item* items, int n, bool capture) {
   if (2 * n > nf3d::RUN_MAX_JOBS) return 0;
   int tiles = 0;
   bool tall = false;
   for (int i = 0; i < n; i++) {
     const nf3d_engine* e = items[i].engine;
     if (e->ep.bt < 2 || e->learned) return 0;  // (a learned PSD is predicted per launch)
+    if (capture && !e->same_launch(*items[0].engine)) return 0;
     tiles += e->noy * e->run_ntx();
     tall = tall || (e->ep.bt == 5 && e->ep.bh >= 48);
   }
@@ -1659,7 +1669,7 @@ void run_batch(const nf3d_run_item* items, int n, hipStream_t s, bool timed, boo
   if (!capture)
     for (int i = 0; i < n; i++) items[i].engine->order_before(s);
   std::vector<nf3d_engine::RangePlan> plans(n);
-  const int pair_frames = pair_runs(items, n);
+  const int pair_frames = pair_runs(items, n, capture);
   for (int i = 0; i < n; i++) {
     const nf3d_run_item& it = items[i];
     plans[i] = it.engine->plan_range(it.first, it.count, it.src, it.src_stride, it.dst, it.dst_stride, pair_frames);
@@ -2247,7 +2257,7 @@ int capture_batch(const nf3d_run_item* items, int n, void* stream, nf3d_graph** 
       }
       // buffers the launches use, allocated outside the capture
       e->plan_range(items[i].first, items[i].count, items[i].src, items[i].src_stride, items[i].dst,
-                    items[i].dst_stride, pair_runs(items, n));
+                    items[i].dst_stride, pair_runs(items, n, true));
     }
     // no profiling events inside the graph
     std::vector<bool> prof(n);

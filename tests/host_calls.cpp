@@ -110,10 +110,16 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
   waits.push_back(Wait{s, recorded[e]});
   return hipSuccess;
 }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorNotSupported; }
-hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, hipGraphNode_t*, char*, size_t) { return hipErrorNotSupported; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+  *g = handle<hipGraph_t>();
+  return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+  *x = handle<hipGraphExec_t>();
+  return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return fresh_event(e); }
@@ -363,6 +369,29 @@ void pairs() {
     }
   }
 }
+
+// Captured batches: pairs only where all engines share their launches.
+void captured_pairs() {
+  Planes P(W, H);
+  for (int second : {16, 24}) {
+    nf3d_engine *a = engine(3), *b = engine(3, second);
+    std::vector<nf3d_run_item> it;
+    for (nf3d_engine* e : {a, b}) it.push_back(nf3d_run_item{e, 0, 20, P.src.data(), W, P.dst.data(), W});
+    nf3d_graph* g = nullptr;
+    char err[256] = {0};
+    run_jobs.clear();
+    CHECK(nf3d_run_device_batch_graph(it.data(), 2, stream(1), &g, err, sizeof err) == 0);
+    // (18 whole windows a plane: pairs of 9 frames, or launches of 9)
+    CHECK(run_jobs == (second == 16 ? std::vector<int>{4} : std::vector<int>(4, 1)));
+    CHECK(nf3d_graph_launch(g, stream(1)) == 0);
+    nf3d_graph_destroy(g);
+    run_jobs.clear();
+    batch({a, b}, P, 0, 20, stream(1));
+    CHECK(run_jobs == (second == 16 ? std::vector<int>{4} : std::vector<int>(2, 2)));
+    nf3d_engine_destroy(a);
+    nf3d_engine_destroy(b);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -372,6 +401,7 @@ int main(int argc, char** argv) {
   else if (name == "pinned_refused") pinned_refused();
   else if (name == "engines_part") engines_part();
   else if (name == "pairs") pairs();
+  else if (name == "captured_pairs") captured_pairs();
   else return 2;
   return 0;
 }

@@ -24,7 +24,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["missing_frame", "frame_throws", "pinned_refused", "engines_part", "pairs"])
+@pytest.mark.parametrize("case", ["missing_frame", "frame_throws", "pinned_refused", "engines_part", "pairs", "captured_pairs"])
 def test_host(program, case):
     r = subprocess.run([program, case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
