@@ -862,7 +862,7 @@ struct nf3d_engine {
   void region_psd(const uint8_t* src, long long pitch, int rx, int ry, float* out, hipStream_t s) {
     if (!d_rspec) {
       d_rspec = dev_alloc<float2>(spec_elems);
-      d_rsums = dev_alloc<float>(nb);
+      d_rsums = dev_alloc<float>(nb + 2 * noy);  // and the block rows' minima
     }
     PlaneJob J = base_job();
     J.src = src;
@@ -879,6 +879,8 @@ struct nf3d_engine {
     P.pwin = d_pwin;
     P.degrid = ep.degrid;
     P.sums = d_rsums;
+    P.row_min = d_rsums + nb;
+    P.row_at = reinterpret_cast<int*>(d_rsums + nb + noy);
     check(nf3d::launch_pattern(P, s), "pattern kernels");
     check(nf3d::launch_pattern_regions(P, rx, ry, out, nullptr, 1.0f, s), "region pattern kernel");
   }

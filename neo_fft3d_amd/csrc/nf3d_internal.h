@@ -123,6 +123,8 @@ struct PatternJob {
   int px, py;          // fixed block, or 0,0 = search
   float* pattern2d;    // out [bh*outwidth]
   float* sums;         // scratch [nb]
+  float* row_min;      // scratch [noy] (regions without choice), or null: each block row's first minimum
+  int* row_at;         // ... and its block
   int* choice;         // out [2]: px, py (null: the sums alone)
 };
 

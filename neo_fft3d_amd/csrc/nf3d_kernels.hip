@@ -82,31 +82,30 @@ __global__ void __launch_bounds__(64) k_pattern_sums(PatternJob J) {
   if (l == 0) J.sums[b] = s;
 }
 
-// The first strict minimum below 1e15 of the sums of the search range's
-// blocks in [x0, x1) x [y0, y1), in row-major order (src/helper.cpp:82-88):
-// the smallest value, the first block of equal ones.  256 lanes take the
-// blocks in turn and meet in LDS (one lane alone waited for every load:
-// k_pattern_set took 124 us on 1,856 sums, now 6.7 us).  Returns the block's
-// index by * nox + bx, or -1.
-__device__ __forceinline__ int pattern_search(const PatternJob& J, int x0, int x1, int y0, int y1, float* rv, int* ri) {
-  x0 = max(x0, 2);
-  y0 = max(y0, 2);
-  x1 = min(x1, J.nox - 2);
-  y1 = min(y1, J.noy - 2);
-  const int w = max(x1 - x0, 0), n = w * max(y1 - y0, 0), t = threadIdx.x;
+// The first strict minimum below 1e15 of n candidates in block order, `at(k,
+// value, index)`: the smallest value, the lowest index of equal ones
+// (src/helper.cpp:82-88).  256 lanes take the candidates in turn and meet in
+// LDS (one lane alone waited for every load: k_pattern_set took 124 us on
+// 1,856 sums, now 6.7 us).  Returns the index, 0x7fffffff for none, the value
+// in rv[0].
+constexpr int NO_BLOCK = 0x7fffffff;
+template <class At>
+__device__ __forceinline__ int first_minimum(int n, At at, float* rv, int* ri) {
+  const int t = threadIdx.x;
   float best = 1e15f;
-  int at = 0x7fffffff;
+  int where = NO_BLOCK;
   for (int k = t; k < n; k += 256) {
-    const int y = k / w, i = (y0 + y) * J.nox + x0 + (k - y * w);
-    const float s = J.sums[i];
+    float s;
+    int i;
+    at(k, s, i);
     if (s < best) {
       best = s;
-      at = i;
+      where = i;
     }
   }
   __syncthreads();  // (a second search: the first one's result is read)
   rv[t] = best;
-  ri[t] = at;
+  ri[t] = where;
   __syncthreads();
   int h = 1;
   while (h < min(n, 256)) h <<= 1;  // lanes past n hold no block
@@ -117,7 +116,36 @@ __device__ __forceinline__ int pattern_search(const PatternJob& J, int x0, int x
     }
     __syncthreads();
   }
-  return ri[0] == 0x7fffffff ? -1 : ri[0];
+  return ri[0];
+}
+
+// ... over the sums of the search range's blocks in [x0, x1) x [y0, y1): the
+// block's index by * nox + bx.
+__device__ __forceinline__ int pattern_search(const PatternJob& J, int x0, int x1, int y0, int y1, float* rv, int* ri) {
+  x0 = max(x0, 2);
+  y0 = max(y0, 2);
+  x1 = min(x1, J.nox - 2);
+  y1 = min(y1, J.noy - 2);
+  const int w = max(x1 - x0, 0), n = w * max(y1 - y0, 0);
+  return first_minimum(
+      n,
+      [&](int k, float& s, int& i) {
+        const int y = k / w;
+        i = (y0 + y) * J.nox + x0 + (k - y * w);
+        s = J.sums[i];
+      },
+      rv, ri);
+}
+
+// The search of each block row, for regions that take the whole plane's block.
+__global__ void __launch_bounds__(256) k_pattern_rows(PatternJob J) {
+  __shared__ float rv[256];
+  __shared__ int ri[256];
+  const int y = blockIdx.x, i = pattern_search(J, 0, J.nox, y, y + 1, rv, ri);
+  if (threadIdx.x == 0) {
+    J.row_min[y] = rv[0];
+    J.row_at[y] = i;
+  }
 }
 
 // The searched block, or the given one, and its pattern (src/helper.cpp:
@@ -129,7 +157,7 @@ __global__ void __launch_bounds__(256) k_pattern_set(PatternJob J) {
   int px = J.px, py = J.py;
   if (px == 0 && py == 0) {
     const int i = pattern_search(J, 0, J.nox, 0, J.noy, rv, ri);
-    if (i >= 0) {
+    if (i != NO_BLOCK) {
       py = i / J.nox;
       px = i - py * J.nox;
     }
@@ -150,9 +178,9 @@ __global__ void __launch_bounds__(256) k_pattern_set(PatternJob J) {
 // pattern of its own first strict minimum of the same sums over the blocks
 // of the reference's search range (blocks 2..nox-3, 2..noy-3) that lie in
 // it -- or, for a region with none of them, the block chosen for the whole
-// plane (J.choice, written by k_pattern_set; null: searched here, which for
-// the few such regions costs less than a launch of its own, 6.7 us, before
-// this one).  The pattern goes to every
+// plane: J.choice, written by k_pattern_set; null: the first minimum of the
+// block rows' (J.row_min, written by k_pattern_rows), or without them
+// searched here, see launch_pattern_regions.  The pattern goes to every
 // block of the region: out2d = |X - g G|^2 pwin, out3d = out2d * mult3d
 // (out3d null: out2d alone).  blockIdx.x: the region, blockIdx.y: 256 of the
 // coefficients (1080p at 48x48 in regions of 4 x 4 has 144 regions, fewer
@@ -166,7 +194,15 @@ __global__ void __launch_bounds__(256) k_pattern_regions(PatternJob J, int rx, i
   const int qy = blockIdx.x / nqx, qx = blockIdx.x - qy * nqx;
   const int x0 = qx * rx, x1 = min(J.nox, x0 + rx), y0 = qy * ry, y1 = min(J.noy, y0 + ry);
   int c = pattern_search(J, x0, x1, y0, y1, rv, ri);
-  if (c < 0) c = J.choice ? J.choice[1] * J.nox + J.choice[0] : max(pattern_search(J, 0, J.nox, 0, J.noy, rv, ri), 0);
+  if (c == NO_BLOCK) {  // (uniform)
+    if (J.choice)
+      c = J.choice[1] * J.nox + J.choice[0];
+    else if (J.row_min)
+      c = first_minimum(J.noy, [&](int k, float& v, int& i) { v = J.row_min[k]; i = J.row_at[k]; }, rv, ri);
+    else
+      c = pattern_search(J, 0, J.nox, 0, J.noy, rv, ri);
+    if (c == NO_BLOCK) c = 0;
+  }
   const int n = J.bh * J.outwidth;
   const int k = blockIdx.y * 256 + threadIdx.x;
   if (k >= n) return;
@@ -243,12 +279,30 @@ hipError_t launch_pattern(const PatternJob& J, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Blocks of a plane past which regions without a block of the search range
+// take the plane's from the block rows' minima instead of each searching the
+// plane: the rows' launch costs 2 us, a search one more for every 3,000 blocks
+// and all the border regions' searches together the caches' rate.  Whole call,
+// search and rows: 2,310 blocks 22 and 23 us, 3,726 72 and 73 (in regions of one
+// block 90 and 87), 8,349 59 and 57, 32,776 76 and 59, 519,901 of 8x8 in regions
+// of one block (5,992 of them on the border) 2,516 and 660.
+constexpr int REGION_SCAN = 4096;
 hipError_t launch_pattern_regions(const PatternJob& J, int rx, int ry, float* out2d, float* out3d, float mult3d,
                                   hipStream_t s) {
   if (rx < 1 || ry < 1) return hipErrorInvalidValue;
-  const int nq = ((J.nox + rx - 1) / rx) * ((J.noy + ry - 1) / ry);
+  const int nqx = (J.nox + rx - 1) / rx, nqy = (J.noy + ry - 1) / ry, nq = nqx * nqy;
   const int nk = (J.bh * J.outwidth + 255) / 256;
-  hipLaunchKernelGGL(k_pattern_regions, dim3(nq, nk), dim3(256), 0, s, J, rx, ry, out2d, out3d, mult3d);
+  PatternJob P = J;
+  if (!J.choice && J.row_min) {
+    // regions without a block of the search range, those of the plane's
+    // border: region columns (rows) with one have a block in [2, n - 2)
+    auto searched = [](int n, int r) { return n > 4 ? (n - 3) / r - 2 / r + 1 : 0; };
+    if (J.nox * J.noy > REGION_SCAN && searched(J.nox, rx) * searched(J.noy, ry) < nq)
+      hipLaunchKernelGGL(k_pattern_rows, dim3(J.noy), dim3(256), 0, s, J);
+    else
+      P.row_min = nullptr;
+  }
+  hipLaunchKernelGGL(k_pattern_regions, dim3(nq, nk), dim3(256), 0, s, P, rx, ry, out2d, out3d, mult3d);
   return hipGetLastError();
 }
 
