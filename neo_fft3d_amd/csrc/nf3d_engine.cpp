@@ -423,7 +423,7 @@ struct nf3d_engine {
   }
 
   // Spectrum of block (0,0) of a constant maximum-value cover without chroma
-  // centring (src/fft3d_engine.h:384-404), with the gather's float products
+  // centring (src/fft3d_engine.h:384-404), with the reference's float products
   // (corner block: top rows (wx*wy)*p or (wy*p)*wx, band rows (wx*p)*wy) and a
   // double-precision DFT rounded once to float.
   void build_grid() {

@@ -24,7 +24,7 @@ __device__ __forceinline__ float pattern_term(float2 c, float2 g, float gcur, fl
 // the reference's sequential float order (src/helper.cpp:57-89).  A wavefront
 // per block: its 64 lanes read the spectrum, the gridsample and the pattern
 // window row by row of 64 coefficients (coalesced, the next PS_ROWS rows in
-// flight) and leave the terms in LDS; one lane then adds them in order, 16
+// flight) and leave the terms in LDS; every lane then adds them in order, 16
 // bytes a read.  Bound by that serial chain of bh * (bw/2+1) adds, which the
 // blocks' wavefronts (two to three per SIMD at 1080p) run side by side; with
 // a lane per block instead, every load was a line of its own and the few

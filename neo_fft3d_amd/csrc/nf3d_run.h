@@ -428,7 +428,8 @@ __device__ __forceinline__ void split_combine_inv(float2 (&c)[N / 2], int h) {
 // place of the row and column FFTs.  With two lanes a column and rolled tile
 // loops it takes 128 / 155 / 188 registers (32 / 48 / 64, bt = 3), so two to
 // four wavefronts share a SIMD: 48/16 on 3840x2160 4:2:0, 8 frames, 3480 us
-// at one wavefront per SIMD with 424 registers, 1800 us now.
+// at one wavefront per SIMD with 424 registers, 1800 us with that change alone,
+// 1600 now.
 //
 // Waves per SIMD the register budget is cut for (LDS allows three workgroups
 // per CU at 48x48): three, or two for the variants whose spectral pass holds
@@ -446,8 +447,8 @@ constexpr int run_waves_per_simd() {
 // RES (Kalman): a lane keeps its elements' state in registers from the first
 // frame of a launch to its last (12 bytes an element: 48 registers at 32x32,
 // 72 at 48x48) instead of reading and writing it for every frame: UHD 4:2:0
-// 10-bit, 11 frames a launch, 8x8 1289 -> 814 us, 16x16 1569 -> 953, 24x24
-// 1530 -> 1092, 32x32 1452 -> 1141, 48x48 1477 -> 1347.  At 64x64 96 more do
+// 10-bit, 11 frames a launch, 8x8 1289 -> 760 us, 16x16 1569 -> 975, 24x24
+// 1530 -> 1080, 32x32 1452 -> 1140, 48x48 1477 -> 1350.  At 64x64 96 more do
 // not fit (344 bytes of scratch a lane: 1649 -> 2437).
 template <int BW, int BH, int NT, int MODE, int BT, int SHP, bool MF = false, bool RES = false>
 __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP, RES>())) k_run(RunBatch B_arg) {
@@ -589,7 +590,7 @@ __global__ void __launch_bounds__(NT, (run_waves_per_simd<BH, MODE, BT, SHP, RES
       // wavefront, highest blocks first.  Spectral block b overlaps only the
       // gather stage of blocks b and b+1 (static_assert below), so a round
       // writes over stages its own round or earlier rounds have read, and one
-      // barrier per round (operands loaded by both wavefronts) is enough.
+      // barrier per round (operands loaded by every wavefront) is enough.
       static_assert(BW == BH && (BW == 32 || BW == 48 || BW == 64), "matrix-core DFT: 32x32, 48x48 or 64x64 blocks");
       static_assert(LSPEC >= LA && 2 * LA - LSPEC >= (BPW - 1) * (LSPEC - LA), "spectra overlap stages b, b+1 only");
       constexpr int NW = NT / 64, MB = (BPW + NW - 1) / NW;
