@@ -143,7 +143,9 @@ int nf3d_run_host_batch(const nf3d_run_item* items, int n, char* err, size_t err
  * `stream` (a non-null hipStream_t) instead of being run; nf3d_graph_launch
  * replays it on a stream (each replay filters the same frames again, as a
  * repeated batch call would).  Capture needs the engines' pattern estimate
- * already made (a first, uncaptured call does it) since it synchronises. */
+ * already made (a first, uncaptured call does it) since it synchronises.  A
+ * batch of several block shapes is best captured after an uncaptured call of
+ * it, the form in which such graphs are tested. */
 typedef struct nf3d_graph nf3d_graph;
 int nf3d_run_device_batch_graph(const nf3d_run_item* items, int n, void* stream, nf3d_graph** graph, char* err,
                                 size_t errlen);
